@@ -130,11 +130,65 @@ __device__ __forceinline__ void load_block_h(const uint32_t* M, int d, int I, fl
     v[8] = lo_half(p[4 * len], (H*)nullptr);
 }
 
-// wave64 butterfly sum
+// Butterfly sums over a wave without LDS: the lanes exchange through
+// v_permlane32/16_swap (lane ^ 32, lane ^ 16: the two results of a swap of x
+// with itself are the two halves', rows', values in every lane) and DPP moves
+// (row_ror:8 is lane ^ 8; with the values then equal at lane ^ 8, row_ror:4
+// is lane ^ 4; quad_perm for 2 and 1), so the order of the sum is that of
+// __shfl_xor's 32, 16, ..., 1.  A __shfl_xor of a double is two ds_bpermute,
+// six dependent LDS round trips per sum; the iteration kernels of small
+// systems spent 0.5 us of their 3-6 us in each block-wide sum.
+__device__ __forceinline__ uint32_t lane_xor32(uint32_t x, uint32_t& other)
+{
+    const auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+    other = r[1];
+    return r[0];
+}
+__device__ __forceinline__ uint32_t lane_xor16(uint32_t x, uint32_t& other)
+{
+    const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+    other = r[1];
+    return r[0];
+}
+constexpr int kDppRor8 = 0x128, kDppRor4 = 0x124, kDppXor2 = 0x4e, kDppXor1 = 0xb1;
+template <int CTRL>
+__device__ __forceinline__ float dpp_move(float v)
+{
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(double v)
+{
+    return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, true),
+                            __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, true));
+}
 __device__ __forceinline__ double wave_sum(double v)
 {
-#pragma unroll
-    for(int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    uint32_t bh, bl;
+    uint32_t ah = lane_xor32((uint32_t)__double2hiint(v), bh), al = lane_xor32((uint32_t)__double2loint(v), bl);
+    v = __hiloint2double((int)ah, (int)al) + __hiloint2double((int)bh, (int)bl);
+    ah = lane_xor16((uint32_t)__double2hiint(v), bh);
+    al = lane_xor16((uint32_t)__double2loint(v), bl);
+    v = __hiloint2double((int)ah, (int)al) + __hiloint2double((int)bh, (int)bl);
+    v += dpp_move<kDppRor8>(v);
+    v += dpp_move<kDppRor4>(v);
+    v += dpp_move<kDppXor2>(v);
+    v += dpp_move<kDppXor1>(v);
+    return v;
+}
+// The same over each group of `width` (16 or 32) lanes.
+__device__ __forceinline__ float group_sum(float v, int width)
+{
+    if(width == 32)
+    {
+        uint32_t b;
+        const uint32_t a = lane_xor16(__float_as_uint(v), b);
+        v = __uint_as_float(a) + __uint_as_float(b);
+    }
+    v += dpp_move<kDppRor8>(v);
+    v += dpp_move<kDppRor4>(v);
+    v += dpp_move<kDppXor2>(v);
+    v += dpp_move<kDppXor1>(v);
     return v;
 }
 
@@ -148,6 +202,18 @@ __device__ double block_sum(double v, double* smem)
     double t = 0.0;
     for(int w = 0; w < (int)(blockDim.x + 63) / 64; ++w) t += smem[w];
     __syncthreads();
+    return t;
+}
+
+// block_sum with one barrier: smem (one double per wave) must not be written
+// again before the kernel's next barrier.
+__device__ __forceinline__ double block_sum_once(double v, double* smem)
+{
+    v = wave_sum(v);
+    if((threadIdx.x & 63) == 0) smem[threadIdx.x >> 6] = v;
+    __syncthreads();
+    double t = 0.0;
+    for(int w = 0; w < (int)(blockDim.x + 63) / 64; ++w) t += smem[w];
     return t;
 }
 
@@ -1680,7 +1746,7 @@ __global__ void __launch_bounds__(256) k_precond_finish(DevData d, int force)
 {
     // rows by XCD as in the SpMV (each XCD a contiguous run of workgroups)
     const int wgi = xcd_tile(blockIdx.x, gridDim.x);
-    __shared__ double smem[8];
+    __shared__ double smem[4], smem2[4];
     const int4 w = d.wg_pre[wgi];
     const int  s = d.single ? 0 : w.x;
     SysState&  st = d.state[s];
@@ -1754,7 +1820,7 @@ __global__ void __launch_bounds__(256) k_precond_finish(DevData d, int force)
     }
     if(!force)
     {
-        const double rr = block_sum(share, smem);
+        const double rr = block_sum_once(share, smem);
         int ns = kRunning, fail = kOk, chk = 0;
         if(!st.frozen)
         {
@@ -1813,7 +1879,7 @@ __global__ void __launch_bounds__(256) k_precond_finish(DevData d, int force)
         part = (double)r0 * z0 + (double)r1 * z1 + (double)r2 * z2;
     }
     if(force) return;
-    part = block_sum_last(part, smem);
+    part = block_sum_last(part, smem2);
     if(threadIdx.x == 0) d.part_pre[wgi] = part;
 }
 
@@ -2106,7 +2172,7 @@ __global__ void __launch_bounds__(256) k_spmv_fused(DevData d, const float* __re
     SpmvChunk<U> c;
     const int n0 = min(CH, e1 - e0);
     if(n0 > 0) spmv_load_chunk<U, NT>(d, p_old, e0, n0, c);
-    const double rz = block_sum(share, smem);
+    const double rz = block_sum_once(share, smem);  // barriers follow before smem is used again
     const bool bad = !finite_d(rz) || (st_rule == kRuleTrueRel && rz <= 0.0);
     if(wg == wg_range(d, d.wg_spmv_range, d.n_wg_spmv, s).x && threadIdx.x == 0)
     {
@@ -2246,7 +2312,7 @@ __global__ void __launch_bounds__(256) k_update(DevData d, const float* __restri
 {
     // rows by XCD as in the SpMV (each XCD a contiguous run of workgroups)
     const int wgi = xcd_tile(blockIdx.x, gridDim.x);
-    __shared__ double smem[8];
+    __shared__ double smem[8], smem2[4];
     const int4 w = d.wg_upd[wgi];
     const int  s = d.single ? 0 : w.x;
     SysState&  st = d.state[s];
@@ -2338,7 +2404,7 @@ __global__ void __launch_bounds__(256) k_update(DevData d, const float* __restri
     float alpha = 0.f;
     if(mode == 0)
     {
-        const double pAp = block_sum(share, smem);
+        const double pAp = block_sum_once(share, smem);
         const bool bad = !finite_d(pAp) || (st.rule == kRuleTrueRel && pAp <= 0.0);
         if((int)wgi == wg_range(d, d.wg_upd_range, d.n_wg_upd, s).x && threadIdx.x == 0)
         {
@@ -2396,12 +2462,9 @@ __global__ void __launch_bounds__(256) k_update(DevData d, const float* __restri
             const int      parent = __shfl(my_parent, gbase + (c - cb), 64);
             const bool in = (mask >> lane) & 1u;
             float sx = in ? r0 : 0.f, sy = in ? r1 : 0.f, sz = in ? r2 : 0.f;
-            for(int off = d.bank >> 1; off > 0; off >>= 1)
-            {
-                sx += __shfl_xor(sx, off, 64);
-                sy += __shfl_xor(sy, off, 64);
-                sz += __shfl_xor(sz, off, 64);
-            }
+            sx = group_sum(sx, d.bank);
+            sy = group_sum(sy, d.bank);
+            sz = group_sum(sz, d.bank);
             if(lane == 0)
             {
                 const long long pc = 3 * (long long)parent;
@@ -2415,7 +2478,7 @@ __global__ void __launch_bounds__(256) k_update(DevData d, const float* __restri
     // the r.r partial of each wave goes to LDS ahead of the barrier the deeper
     // partials need; thread 0 adds the four after it
     part = wave_sum(part);
-    if((threadIdx.x & 63) == 0) smem[threadIdx.x >> 6] = part;
+    if((threadIdx.x & 63) == 0) smem2[threadIdx.x >> 6] = part;
     __syncthreads();
     // one partial per deeper ancestor of the group's components (levels >= 2),
     // summed over the components in order
@@ -2423,15 +2486,27 @@ __global__ void __launch_bounds__(256) k_update(DevData d, const float* __restri
     {
         for(int t = threadIdx.x; t < grp.y; t += blockDim.x)
         {
+            // four components' LDS reads in flight at a time (one at a time
+            // was 1.5-2 us of the kernel's 6 on a small system)
+            constexpr int K = 4;
             float ax = 0.f, ay = 0.f, az = 0.f;
-            for(int c = grp.z; c < grp.w; ++c)
+            for(int c = grp.z; c < grp.w; c += K)
             {
-                const int4 ds = sDs[c - grp.z];
-                if(ds.x == t || ds.y == t || ds.z == t || ds.w == t)
+                int4  ds[K];
+                float v[K][3];
+#pragma unroll
+                for(int k = 0; k < K; ++k)
                 {
-                    const int j = c - grp.z;
-                    ax += sC[3 * j]; ay += sC[3 * j + 1]; az += sC[3 * j + 2];
+                    const int j = min(c + k, grp.w - 1) - grp.z;
+                    ds[k] = sDs[j];
+                    v[k][0] = sC[3 * j]; v[k][1] = sC[3 * j + 1]; v[k][2] = sC[3 * j + 2];
                 }
+#pragma unroll
+                for(int k = 0; k < K; ++k)
+                    if(c + k < grp.w && (ds[k].x == t || ds[k].y == t || ds[k].z == t || ds[k].w == t))
+                    {
+                        ax += v[k][0]; ay += v[k][1]; az += v[k][2];
+                    }
             }
             const long long o = 3 * (long long)(grp.x + t);
             d.part_deep[o] = ax; d.part_deep[o + 1] = ay; d.part_deep[o + 2] = az;
@@ -2440,7 +2515,7 @@ __global__ void __launch_bounds__(256) k_update(DevData d, const float* __restri
     if(threadIdx.x == 0)
     {
         double t = 0.0;
-        for(int w = 0; w < (int)(blockDim.x + 63) / 64; ++w) t += smem[w];
+        for(int w = 0; w < (int)(blockDim.x + 63) / 64; ++w) t += smem2[w];
         d.part_upd[wgi] = t;
     }
 }
