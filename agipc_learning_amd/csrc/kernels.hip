@@ -2599,56 +2599,90 @@ __global__ void __launch_bounds__(256) k_check_finish(DevData d, int report_only
 
 // ================================================================ FP64 API
 
-// y_int = A x_int (FP64 full block CSR over the FP64 input blocks).
-__global__ void __launch_bounds__(256) k_spmv64(DevData d, const double* x, double* y)
+// x in the internal row order (padding rows zero).
+__global__ void __launch_bounds__(256) k_rows_from_ext64(const int* __restrict__ int_to_ext,
+                                                         const double* __restrict__ src_ext,
+                                                         double* __restrict__ dst_int, int n_rows)
 {
-    const int row = blockIdx.x * blockDim.x + threadIdx.x;
-    if(row >= d.n_rows) return;
-    double a0 = 0.0, a1 = 0.0, a2 = 0.0;
-    for(int e = d.row_ptr[row]; e < d.row_ptr[row + 1]; ++e)
-    {
-        const int code = d.entry_src[e];
-        const double* B = d.vals64 + 9 * (long long)(code & 0x7fffffff);
-        const long long c = 3 * (long long)d.col[e];
-        const double x0 = x[c], x1 = x[c + 1], x2 = x[c + 2];
-        if(code >= 0)
-        {
-            a0 += B[0] * x0 + B[3] * x1 + B[6] * x2;
-            a1 += B[1] * x0 + B[4] * x1 + B[7] * x2;
-            a2 += B[2] * x0 + B[5] * x1 + B[8] * x2;
-        }
-        else
-        {
-            a0 += B[0] * x0 + B[1] * x1 + B[2] * x2;
-            a1 += B[3] * x0 + B[4] * x1 + B[5] * x2;
-            a2 += B[6] * x0 + B[7] * x1 + B[8] * x2;
-        }
-    }
-    y[3 * (long long)row] = a0;
-    y[3 * (long long)row + 1] = a1;
-    y[3 * (long long)row + 2] = a2;
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;  // one value each: whole lines per store
+    if(i >= 3 * n_rows) return;
+    const int row = i / 3, e = int_to_ext[row];
+    dst_int[i] = e >= 0 ? src_ext[3 * (long long)e + (i - 3 * row)] : 0.0;
 }
 
-__global__ void __launch_bounds__(256) k_gather_ext64(const int* ext_to_int, const double* src_ext, double* dst_int,
-                                                      int n_ext)
+// y_ext = a A x_int + b y_ext (FP64 full block CSR over the FP64 input blocks).
+// A workgroup owns 64 consecutive rows; three lanes share an entry, lane q
+// forming component q of its product, so a wave instruction reads 21 blocks
+// of 72 contiguous bytes (a row's own upper blocks follow each other) instead
+// of 64 lanes 72 bytes apart.  The products pass through LDS and three
+// threads per row add the row's in entry order; a workgroup whose rows hold
+// more than a chunk takes several chunks.  Bound by the blocks' bytes, each
+// read for its row and, transposed, for its column (the second mostly from
+// the caches: rows run in Morton order and each XCD has a contiguous run).
+// 226,981 rows, 1.77 M upper blocks: one thread per row 134 us.
+constexpr int kRows64 = 64, kEntries64 = 85 * 12;
+__global__ void __launch_bounds__(256) k_spmv64(DevData d, const int* __restrict__ int_to_ext,
+                                                const double* __restrict__ x, double a, double b,
+                                                double* __restrict__ y)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if(i >= n_ext) return;
-    const long long R = ext_to_int[i];
-    for(int c = 0; c < 3; ++c) dst_int[3 * R + c] = src_ext[3 * (long long)i + c];
-}
-
-__global__ void __launch_bounds__(256) k_axpby_int_to_ext(const int* ext_to_int, const double* y_int, double* y_ext,
-                                                          double a, double b, int n_ext)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if(i >= n_ext) return;
-    const long long R = ext_to_int[i];
-    for(int c = 0; c < 3; ++c)
+    constexpr int K = 4;  // entries in flight per thread
+    static_assert(kEntries64 % (85 * K) == 0, "whole passes");
+    __shared__ double sP[3 * kEntries64];
+    const int tid = threadIdx.x;
+    const int r0 = xcd_tile(blockIdx.x, gridDim.x) * kRows64, r1 = min(r0 + kRows64, d.n_rows);
+    const int e0 = d.row_ptr[r0], e1 = d.row_ptr[r1];
+    const int own = r0 + tid / 3, q = tid % 3;  // thread's row and component; as a worker, entry tid / 3 of a pass
+    const bool has_row = tid < 3 * kRows64 && own < r1;
+    const int rb = has_row ? d.row_ptr[own] : 0, re = has_row ? d.row_ptr[own + 1] : 0;
+    double acc = 0.0;
+#pragma unroll 1
+    for(int base = e0; base < e1; base += kEntries64)
     {
-        const long long o = 3 * (long long)i + c;
-        y_ext[o] = a * y_int[3 * R + c] + (b != 0.0 ? b * y_ext[o] : 0.0);
+        const int n = min(kEntries64, e1 - base);
+#pragma unroll 1
+        for(int pass = tid / 3; pass < n && tid < 255; pass += 85 * K)
+        {
+            int    code[K], col[K];
+            double v[K][3], xv[K][3];
+#pragma unroll
+            for(int k = 0; k < K; ++k)
+            {
+                const int e = base + min(pass + 85 * k, n - 1);
+                code[k] = d.entry_src[e];
+                col[k]  = d.col[e];
+            }
+#pragma unroll
+            for(int k = 0; k < K; ++k)
+            {
+                // component q of B x: row q of a block kept as is, column q of a transposed one
+                const double* B = d.vals64 + 9 * (long long)(code[k] & 0x7fffffff) + (code[k] >= 0 ? q : 3 * q);
+                const int step = code[k] >= 0 ? 3 : 1;
+                const double* xc = x + 3 * (long long)col[k];
+#pragma unroll
+                for(int c = 0; c < 3; ++c)
+                {
+                    v[k][c]  = B[c * step];
+                    xv[k][c] = xc[c];
+                }
+            }
+#pragma unroll
+            for(int k = 0; k < K; ++k)
+                if(pass + 85 * k < n)
+                    sP[3 * (pass + 85 * k) + q] = v[k][0] * xv[k][0] + v[k][1] * xv[k][1] + v[k][2] * xv[k][2];
+        }
+        __syncthreads();
+        if(has_row)
+        {
+            const int hi = min(re, base + n) - base;
+            for(int e = max(rb, base) - base; e < hi; ++e) acc += sP[3 * e + q];
+        }
+        __syncthreads();
     }
+    if(!has_row) return;
+    const int ext = int_to_ext[own];
+    if(ext < 0) return;  // padding row
+    const long long o = 3 * (long long)ext + q;
+    y[o] = a * acc + (b != 0.0 ? b * y[o] : 0.0);
 }
 
 __global__ void __launch_bounds__(256) k_z32_to_ext(const int* ext_to_int, const float* z, double* dst_ext, int n_ext)
@@ -2992,28 +3026,20 @@ hipError_t launch_true_residual(const DevData& d, int n_wg, int report_only, hip
     return hipSuccess;
 }
 
-hipError_t launch_spmv64(const DevData& d, const double* x, double* y, hipStream_t st)
+hipError_t launch_rows_from_ext64(const int* i2e, const double* src, double* dst, int n_rows, hipStream_t st)
 {
-    if(d.n_rows <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_spmv64, dim3(blocks_for(d.n_rows, 256)), dim3(256), 0, st, d, x, y);
+    if(n_rows == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_rows_from_ext64, dim3(blocks_for(3 * (long long)n_rows, 256)), dim3(256), 0, st, i2e, src, dst,
+                       n_rows);
     MASX_CHECK_LAUNCH();
     return hipSuccess;
 }
 
-hipError_t launch_gather_ext64(const int* e2i, const double* src, double* dst, int n_ext, hipStream_t st)
+hipError_t launch_spmv64(const DevData& d, const int* i2e, const double* x, double a, double b, double* y,
+                         hipStream_t st)
 {
-    if(n_ext <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_gather_ext64, dim3(blocks_for(n_ext, 256)), dim3(256), 0, st, e2i, src, dst, n_ext);
-    MASX_CHECK_LAUNCH();
-    return hipSuccess;
-}
-
-hipError_t launch_axpby_int_to_ext(const int* e2i, const double* y_int, double* y_ext, double a, double b, int n_ext,
-                                   hipStream_t st)
-{
-    if(n_ext <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_axpby_int_to_ext, dim3(blocks_for(n_ext, 256)), dim3(256), 0, st, e2i, y_int, y_ext, a, b,
-                       n_ext);
+    if(d.n_rows == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_spmv64, dim3(blocks_for(d.n_rows, kRows64)), dim3(256), 0, st, d, i2e, x, a, b, y);
     MASX_CHECK_LAUNCH();
     return hipSuccess;
 }

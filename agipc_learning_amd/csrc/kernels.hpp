@@ -53,10 +53,10 @@ hipError_t launch_update(const DevData& d, int n_wg, const float* p, int mode, h
                          const LaunchEvents* ev = nullptr);
 // true residual of the checked (or, report_only, all) systems and its decision
 hipError_t launch_true_residual(const DevData& d, int n_wg, int report_only, hipStream_t st);
-hipError_t launch_spmv64(const DevData& d, const double* x, double* y, hipStream_t st);
-hipError_t launch_gather_ext64(const int* e2i, const double* src, double* dst, int n_ext, hipStream_t st);
-hipError_t launch_axpby_int_to_ext(const int* e2i, const double* y_int, double* y_ext, double a, double b, int n_ext,
-                                   hipStream_t st);
+// rows of x in the internal order (zeros in padding rows), then y = a A x + b y for external rows
+hipError_t launch_rows_from_ext64(const int* i2e, const double* src, double* dst, int n_rows, hipStream_t st);
+hipError_t launch_spmv64(const DevData& d, const int* i2e, const double* x, double a, double b, double* y,
+                         hipStream_t st);
 hipError_t launch_z32_to_ext(const int* e2i, const float* z, double* dst, int n_ext, hipStream_t st);
 hipError_t launch_gather_blocks(const double* src, const uint32_t* idx, double* dst, long long n, hipStream_t st);
 

@@ -394,8 +394,7 @@ void Solver::setup()
     d_E_.alloc(9 * (size_t)std::max<long long>(P.n_gal, 1));
     const size_t nv = 3 * (size_t)P.n_rows;
     d_b64_.alloc(nv);
-    d_tmp64a_.alloc(nv);
-    d_tmp64b_.alloc(nv);
+    d_tmp64_.alloc(nv);
     for(auto* a : {&d_x_, &d_r_, &d_z_, &d_p0_, &d_p1_, &d_Ap_, &d_rt_}) a->alloc(nv);
     d_Rc_.alloc(3 * (size_t)std::max(P.n_coarse, 1));
     d_Zc_.alloc(3 * (size_t)std::max(P.n_coarse, 1));
@@ -1028,10 +1027,9 @@ void Solver::spmv(double a, const double* d_x, double b, double* d_y, hipStream_
 {
     if(!setup_done_) throw std::runtime_error("setup() must precede spmv()");
     hipStream_t st = enter(user);
-    MASX_HIP(hipMemsetAsync(d_tmp64a_.ptr, 0, 3 * (size_t)plan_.n_rows * sizeof(double), st));
-    MASX_HIP(launch_gather_ext64(d_e2i_.ptr, d_x, d_tmp64a_.ptr, plan_.n_ext, st));
-    MASX_HIP(launch_spmv64(dd_, d_tmp64a_.ptr, d_tmp64b_.ptr, st));
-    MASX_HIP(launch_axpby_int_to_ext(d_e2i_.ptr, d_tmp64b_.ptr, d_y, a, b, plan_.n_ext, st));
+    // x leaves the caller's buffer first: x and y may be the same
+    MASX_HIP(launch_rows_from_ext64(d_i2e_.ptr, d_x, d_tmp64_.ptr, plan_.n_rows, st));
+    MASX_HIP(launch_spmv64(dd_, d_i2e_.ptr, d_tmp64_.ptr, a, b, d_y, st));
     leave(user);
 }
 

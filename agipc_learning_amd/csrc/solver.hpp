@@ -179,7 +179,7 @@ class Solver
     void download_device_structures();  // for the host analysis
     int inv_map_key_ = -1;
     DeviceArray<float>     d_vals32_;
-    DeviceArray<double>    d_vals64_, d_E_, d_b64_, d_tmp64a_, d_tmp64b_;
+    DeviceArray<double>    d_vals64_, d_E_, d_b64_, d_tmp64_;
     DeviceArray<float>     d_x_, d_r_, d_z_, d_p0_, d_p1_, d_Ap_, d_rt_, d_Rc_, d_Zc_, d_part_deep_;
     DeviceArray<char>      d_minv_;
     DeviceArray<float>     d_minv_scale_;
