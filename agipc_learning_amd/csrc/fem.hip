@@ -11,8 +11,10 @@
 // structure gives the derivative of the projected matrix in closed form for
 // the parameter gradient (divided differences of max(., 0) on the 3x3 block).
 //
-// Assembly is deterministic: element matrices go to a scratch array, then one
-// thread per target block sums its contributions in tet order.
+// Assembly is deterministic: element matrices go to a scratch array, then
+// every target block's contributions are summed in tet order.  Both kernels
+// move the 720 B per tet in whole lines through LDS: the scratch keeps the
+// ten blocks of 64 consecutive tets block by block (elem_slot).
 #include "fem.hpp"
 
 #include <algorithm>
@@ -28,6 +30,10 @@ namespace
 constexpr int kBlocksPerTet = 10;  // upper 3x3 blocks (a <= b) of a 12x12 element matrix
 
 __host__ __device__ constexpr int tet_block(int a, int b) { return 4 * a - a * (a - 1) / 2 + (b - a); }
+
+// Scratch position (in blocks of 9 doubles) of block k of tet t: the 64 tets of
+// a wave have their k-th blocks side by side.
+__host__ __device__ constexpr int elem_slot(int t, int k) { return ((t >> 6) * kBlocksPerTet + k) * 64 + (t & 63); }
 
 // One Jacobi rotation annihilating A[p][q]; Q accumulates the eigenvectors (columns).
 __device__ __forceinline__ void jrot(double A[3][3], double Q[3][3], int p, int q)
@@ -172,6 +178,13 @@ __device__ void svd3(const double F[3][3], double U[3][3], double S[3], double V
     }
 }
 
+// LDS written by the wave's lanes is readable by all of them after this
+__device__ __forceinline__ void wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // Per-tet quantities shared by the element matrix and the gradient.
 struct TetFrame
 {
@@ -224,13 +237,21 @@ __device__ void tet_frame(const double* __restrict__ Fg, const double* __restric
         for(int j = 0; j < 3; ++j) T.Gh[a][j] = G[a][0] * V[0][j] + G[a][1] * V[1][j] + G[a][2] * V[2][j];
 }
 
+// One thread per tet.  A thread's own 72-byte blocks would be stored 8 bytes
+// at a time, 64 lanes 720 bytes apart (the kernel took 408 us for 1.3 M tets);
+// a wave turns each of the ten blocks over in LDS and stores 4,608 contiguous
+// bytes.
 __global__ void __launch_bounds__(256) k_fem_element(int n_tets, const double* __restrict__ dminv,
                                                      const double* __restrict__ vol, const double* __restrict__ Fg,
                                                      const double* __restrict__ mu, const double* __restrict__ lambda,
                                                      double* __restrict__ elem)
 {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if(t >= n_tets) return;
+    __shared__ double sE[4][64 * 9];
+    const int lane = threadIdx.x & 63;
+    const int t0 = blockIdx.x * blockDim.x + (int)(threadIdx.x & ~63u);  // the wave's first tet
+    if(t0 >= n_tets) return;
+    double* sW = sE[threadIdx.x >> 6];
+    const int t = min(t0 + lane, n_tets - 1);  // the last wave's spare lanes repeat its last tet
     TetFrame T;
     tet_frame(Fg + 9 * (long long)t, dminv + 9 * (long long)t, mu[t], lambda[t], T);
     // projected Hessian in the rotated frame: pair k on (X_ij, X_ji) has
@@ -254,7 +275,6 @@ __global__ void __launch_bounds__(256) k_fem_element(int n_tets, const double* _
             PA[i][j] = acc;
         }
     const double v = vol[t];
-    double* out = elem + (long long)t * kBlocksPerTet * 9;
 #pragma unroll
     for(int a = 0; a < 4; ++a)
 #pragma unroll
@@ -284,44 +304,86 @@ __global__ void __launch_bounds__(256) k_fem_element(int n_tets, const double* _
             for(int i = 0; i < 3; ++i)
 #pragma unroll
                 for(int k = 0; k < 3; ++k) KU[i][k] = Kh[i][0] * T.U[k][0] + Kh[i][1] * T.U[k][1] + Kh[i][2] * T.U[k][2];
-            double* blk = out + 9 * tet_block(a, b);
 #pragma unroll
             for(int i = 0; i < 3; ++i)
 #pragma unroll
                 for(int k = 0; k < 3; ++k)
-                    blk[i + 3 * k] = v * (T.U[i][0] * KU[0][k] + T.U[i][1] * KU[1][k] + T.U[i][2] * KU[2][k]);
+                    sW[9 * lane + i + 3 * k] =
+                        v * (T.U[i][0] * KU[0][k] + T.U[i][1] * KU[1][k] + T.U[i][2] * KU[2][k]);
+            wave_sync();
+            double* out = elem + 9 * (long long)elem_slot(t0, tet_block(a, b));
+#pragma unroll
+            for(int q = 0; q < 9; ++q) out[lane + 64 * q] = sW[lane + 64 * q];
+            wave_sync();
         }
 }
 
+// vals = base + contributions in tet order.  A workgroup owns 64 target blocks
+// and walks their contributions (consecutive in the list) in chunks: nine
+// lanes read one contribution's 72 contiguous bytes (in the transposed order
+// where it is used transposed) into LDS, then the 576 target values are summed
+// from there.  The work is even whatever a block's count (24 on a diagonal, 4-6
+// off it), and each XCD walks a contiguous run of targets.  One thread per
+// target block took 716 us for 13 M contributions of 1.3 M tets.
+constexpr int kGatherTargets = 64, kGatherChunk = 28 * 18;
 __global__ void __launch_bounds__(256) k_fem_gather(long long nb, const long long* __restrict__ ptr,
                                                     const int* __restrict__ contrib, const double* __restrict__ elem,
                                                     const double* __restrict__ base, double* __restrict__ vals)
 {
-    const long long j = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-    if(j >= nb) return;
-    double acc[9];
+    constexpr int K = 6, OWN = (9 * kGatherTargets + 255) / 256;  // contributions in flight and sums per thread
+    static_assert(kGatherChunk % (28 * K) == 0, "whole passes");
+    __shared__ double sE[9 * kGatherChunk];
+    const int tid = threadIdx.x;
+    const int per = (int)(gridDim.x >> 3), rem = (int)(gridDim.x & 7), xcd = (int)(blockIdx.x & 7);
+    const long long j0 = (long long)(xcd * per + min(xcd, rem) + (int)(blockIdx.x >> 3)) * kGatherTargets;
+    const int nj = (int)min((long long)kGatherTargets, nb - j0);
+    const long long e0 = ptr[j0], e1 = ptr[j0 + nj];
+    double acc[OWN];
+    int    lo[OWN], hi[OWN];  // the sums' contributions, relative to e0
 #pragma unroll
-    for(int q = 0; q < 9; ++q) acc[q] = base ? base[9 * j + q] : 0.0;
-    const long long e0 = ptr[j], e1 = ptr[j + 1];
-    for(long long e = e0; e < e1; ++e)
+    for(int m = 0; m < OWN; ++m)
     {
-        const int code = contrib[e];
-        const double* b = elem + (long long)(code >> 1) * 9;
-        if(code & 1)
+        const int o = tid + 256 * m;
+        acc[m] = 0.0;
+        lo[m] = hi[m] = 0;
+        if(o < 9 * nj)
         {
-#pragma unroll
-            for(int i = 0; i < 3; ++i)
-#pragma unroll
-                for(int m = 0; m < 3; ++m) acc[i + 3 * m] += b[m + 3 * i];
-        }
-        else
-        {
-#pragma unroll
-            for(int q = 0; q < 9; ++q) acc[q] += b[q];
+            if(base) acc[m] = base[9 * j0 + o];
+            lo[m] = (int)(ptr[j0 + o / 9] - e0);
+            hi[m] = (int)(ptr[j0 + o / 9 + 1] - e0);
         }
     }
+    const int g = tid / 9, q = tid % 9, qt = q / 3 + 3 * (q % 3);
+    const int total = (int)(e1 - e0);
+#pragma unroll 1
+    for(int c0 = 0; c0 < total; c0 += kGatherChunk)
+    {
+        const int n = min(kGatherChunk, total - c0);
+#pragma unroll 1
+        for(int pass = g; pass < n && tid < 252; pass += 28 * K)
+        {
+            int    code[K];
+            double v[K];
 #pragma unroll
-    for(int q = 0; q < 9; ++q) vals[9 * j + q] = acc[q];
+            for(int k = 0; k < K; ++k) code[k] = contrib[e0 + c0 + min(pass + 28 * k, n - 1)];
+#pragma unroll
+            for(int k = 0; k < K; ++k) v[k] = elem[9 * (long long)(code[k] >> 1) + (code[k] & 1 ? qt : q)];
+#pragma unroll
+            for(int k = 0; k < K; ++k)
+                if(pass + 28 * k < n) sE[9 * (pass + 28 * k) + q] = v[k];
+        }
+        __syncthreads();
+#pragma unroll
+        for(int m = 0; m < OWN; ++m)
+        {
+            const int o = tid + 256 * m, b = max(lo[m], c0) - c0, e = min(hi[m], c0 + n) - c0;
+            for(int k = b; k < e; ++k) acc[m] += sE[9 * k + o % 9];
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for(int m = 0; m < OWN; ++m)
+        if(tid + 256 * m < 9 * nj) vals[9 * j0 + tid + 256 * m] = acc[m];
 }
 
 // g_theta = -vol <Xy, dP[dH/dtheta] Xx> in the rotated frame, Xx = U^T dx G V
@@ -443,7 +505,7 @@ FemHessian::~FemHessian()
 void FemHessian::setup(int n_tets, const int* tets, long long nb, const int* rows, const int* cols)
 {
     if(n_tets <= 0 || !tets) throw std::invalid_argument("no tets");
-    if(n_tets > (1 << 30) / kBlocksPerTet) throw std::invalid_argument("too many tets");
+    if(n_tets > (1 << 30) / kBlocksPerTet - 64) throw std::invalid_argument("too many tets");
     if(nb <= 0 || !rows || !cols) throw std::invalid_argument("empty block structure");
     int n_rows = 0;
     for(long long k = 0; k < nb; ++k)
@@ -499,7 +561,7 @@ void FemHessian::setup(int n_tets, const int* tets, long long nb, const int* row
                 const long long j = find(p, q);
                 if(j < 0) throw std::invalid_argument("a tet edge or vertex has no block in the structure");
                 target.push_back(j);
-                code.push_back(((t * kBlocksPerTet + tet_block(std::min(a, b), std::max(a, b))) << 1) | (a > b ? 1 : 0));
+                code.push_back((elem_slot(t, tet_block(std::min(a, b), std::max(a, b))) << 1) | (a > b ? 1 : 0));
             }
     }
     std::vector<long long> ptr(nb + 1, 0);
@@ -531,7 +593,7 @@ void FemHessian::assemble(const double* dminv, const double* vol, const double* 
 {
     if(n_tets_ <= 0) throw std::runtime_error("fem: setup must come first");
     if(!dminv || !vol || !F || !mu || !lambda || !vals) throw std::invalid_argument("fem: null argument");
-    const size_t need = (size_t)n_tets_ * kBlocksPerTet * 9;
+    const size_t need = ((size_t)n_tets_ + 63) / 64 * 64 * kBlocksPerTet * 9;
     if(need > elem_cap_)
     {
         if(d_elem_) (void)hipFree(d_elem_);
@@ -542,7 +604,7 @@ void FemHessian::assemble(const double* dminv, const double* vol, const double* 
     }
     hipLaunchKernelGGL(k_fem_element, dim3(blocks_of(n_tets_, 256)), dim3(256), 0, st, n_tets_, dminv, vol, F, mu,
                        lambda, d_elem_);
-    hipLaunchKernelGGL(k_fem_gather, dim3(blocks_of(nb_, 256)), dim3(256), 0, st, nb_, d_ptr_, d_contrib_, d_elem_,
+    hipLaunchKernelGGL(k_fem_gather, dim3(blocks_of(nb_, kGatherTargets)), dim3(256), 0, st, nb_, d_ptr_, d_contrib_, d_elem_,
                        base, vals);
     fem_check(hipGetLastError());
 }

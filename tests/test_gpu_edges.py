@@ -52,3 +52,30 @@ def test_spmv64_row_tiles_and_chunks(oracle, n, per_row, hub):
     own = dev(x)
     s.spmv(own, own)
     assert np.linalg.norm(host(own) - want) <= 1e-13 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("n_tets", [1, 63, 64, 65, 190])
+def test_fem_assemble_tet_groups_and_chunks(oracle, n_tets):
+    """Assembly around the 64-tet groups and 64-target tiles, and a tile whose
+    contributions exceed a 504-entry chunk (every tet shares two vertices).
+    Bound as in the other assembly tests (two routes of the same 64-bit
+    projection, 1e-11 of the largest value)."""
+    from agipc_learning_amd import adjoint
+
+    rng = np.random.default_rng(n_tets)
+    n = 2 + 2 * n_tets
+    tets = np.stack([np.zeros(n_tets, int), 2 + 2 * np.arange(n_tets), np.full(n_tets, 1), 3 + 2 * np.arange(n_tets)],
+                    1).astype(np.int32)
+    rng.permuted(tets, axis=1, out=tets)  # both orientations of every pair
+    dminv = rng.standard_normal((n_tets, 9))
+    vol, mu, lam = rng.uniform(0.5, 1.5, n_tets), rng.uniform(1, 2, n_tets), rng.uniform(1, 2, n_tets)
+    F = np.eye(3).reshape(9) + 0.4 * rng.standard_normal((n_tets, 9))
+    rows, cols = adjoint.mesh_structure(n, tets)
+    base = rng.standard_normal((len(rows), 9))
+    fem = native.FemHessian(tets, rows, cols)
+    args = [dev(a) for a in (dminv, vol, F, mu, lam)]
+    got, plain = host(fem.assemble(*args, base=dev(base))), host(fem.assemble(*args))
+    A = oracle.fem_assemble_dense(n, tets, dminv, vol, F, mu, lam)
+    want = np.stack([A[3 * r:3 * r + 3, 3 * c:3 * c + 3].reshape(9, order="F") for r, c in zip(rows, cols)])
+    assert np.abs(plain - want).max() <= 1e-11 * np.abs(want).max()
+    assert np.abs(got - base - want).max() <= 1e-11 * np.abs(want).max()
