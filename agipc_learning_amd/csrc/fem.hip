@@ -240,7 +240,8 @@ __device__ void tet_frame(const double* __restrict__ Fg, const double* __restric
 // One thread per tet.  A thread's own 72-byte blocks would be stored 8 bytes
 // at a time, 64 lanes 720 bytes apart (the kernel took 408 us for 1.3 M tets);
 // a wave turns each of the ten blocks over in LDS and stores 4,608 contiguous
-// bytes.
+// bytes.  Nontemporal: the scratch (933 MB there) passes the caches (541 -> 532 us
+// for the whole assembly, now at 4.1 TB/s of its 2.2 GB, near the copy rate).
 __global__ void __launch_bounds__(256) k_fem_element(int n_tets, const double* __restrict__ dminv,
                                                      const double* __restrict__ vol, const double* __restrict__ Fg,
                                                      const double* __restrict__ mu, const double* __restrict__ lambda,
@@ -313,24 +314,27 @@ __global__ void __launch_bounds__(256) k_fem_element(int n_tets, const double* _
             wave_sync();
             double* out = elem + 9 * (long long)elem_slot(t0, tet_block(a, b));
 #pragma unroll
-            for(int q = 0; q < 9; ++q) out[lane + 64 * q] = sW[lane + 64 * q];
+            for(int q = 0; q < 9; ++q) __builtin_nontemporal_store(sW[lane + 64 * q], &out[lane + 64 * q]);
             wave_sync();
         }
 }
 
-// vals = base + contributions in tet order.  A workgroup owns 64 target blocks
+// vals = base + contributions in tet order.  A workgroup owns 32 target blocks
 // and walks their contributions (consecutive in the list) in chunks: nine
 // lanes read one contribution's 72 contiguous bytes (in the transposed order
-// where it is used transposed) into LDS, then the 576 target values are summed
+// where it is used transposed) into LDS, then the 288 target values are summed
 // from there.  The work is even whatever a block's count (24 on a diagonal, 4-6
 // off it), and each XCD walks a contiguous run of targets.  One thread per
-// target block took 716 us for 13 M contributions of 1.3 M tets.
-constexpr int kGatherTargets = 64, kGatherChunk = 28 * 18;
+// target block took 716 us for 13 M contributions of 1.3 M tets.  A chunk is one
+// pass of nine loads per thread and 18 KB of LDS (eight workgroups per CU): the
+// whole assembly 593 us with 64 targets and chunks of three passes, 532 with
+// this; the scratch read with nontemporal loads was slower (584).
+constexpr int kGatherTargets = 32, kGatherChunk = 28 * 9;
 __global__ void __launch_bounds__(256) k_fem_gather(long long nb, const long long* __restrict__ ptr,
                                                     const int* __restrict__ contrib, const double* __restrict__ elem,
                                                     const double* __restrict__ base, double* __restrict__ vals)
 {
-    constexpr int K = 6, OWN = (9 * kGatherTargets + 255) / 256;  // contributions in flight and sums per thread
+    constexpr int K = 9, OWN = (9 * kGatherTargets + 255) / 256;  // contributions in flight and sums per thread
     static_assert(kGatherChunk % (28 * K) == 0, "whole passes");
     __shared__ double sE[9 * kGatherChunk];
     const int tid = threadIdx.x;
