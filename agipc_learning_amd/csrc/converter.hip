@@ -5,11 +5,19 @@
 // Instead of a global radix sort of (row << 32 | col) keys, triplets are
 // bucketed by block row (integer histogram, scan, scatter) and each row's
 // bucket -- a few dozen entries for a mesh -- is ordered by (col, input
-// index) with a rank sort in LDS, one wavefront per row.  The order inside a
-// duplicate group is the input order, so every sum is formed in a fixed order
-// and the output is bit-reproducible.
+// index) with a rank sort in registers, one wavefront per row (longer rows in
+// LDS).  The order inside a duplicate group is the input order, so every sum
+// is formed in a fixed order and the output is bit-reproducible.
+//
+// Bound by the values (72 B per triplet and per unique block) and, before
+// them, by the atomics of the histogram.  4.04 M triplets in element order,
+// 591 k unique blocks, in this form (and with an atomic per triplet in the count and
+// the scatter, a sort in LDS and a thread per unique block): count 36 (148),
+// scatter 16 (230), row sort 65 (148), sums 107 us (319), 3.3 TB/s of their
+// bytes.
 #include "converter.hpp"
 
+#include <algorithm>
 #include <stdexcept>
 #include <string>
 
@@ -20,34 +28,68 @@ namespace
 constexpr int kScanBlock = 256;
 constexpr int kScanItems = 8;               // elements per thread in the block scan
 constexpr int kScanTile  = kScanBlock * kScanItems;
+constexpr int kRowRegs   = 128;             // longest row sorted in registers (two keys per lane)
 constexpr int kRowCap    = 1024;            // longest row sorted in LDS; longer rows sort in global scratch
+constexpr int kLongGrid  = 1024;            // workgroups that walk the rows longer than kRowRegs
+constexpr uint32_t kHead = 0x80000000u;     // bucket entry: first of its column run (an input index has 31 bits)
+constexpr uint32_t kNone = 0xffffffffu;     // rank of a triplet that is dropped
 
 enum ConvFlag : int { kBadIndex = 1 };
 
-__global__ void __launch_bounds__(256) k_conv_count(int n, int nr, const int* rows, const int* cols, int drop_lower,
-                                                    int* row_count, int* flag)
+// Counts the triplets of every row and gives each its place in its row's
+// bucket (its arrival there: any order will do, the sort below fixes it), so
+// the scatter needs no atomics of its own.  Lanes of a wave with the same row
+// (element order repeats a tet's rows) share one atomic; after kMerge
+// distinct rows the rest take one each, and all of a wave's atomics go out
+// in one instruction.
+constexpr int kMerge = 24;
+__global__ void __launch_bounds__(256) k_conv_count(int n, int nr, const int* __restrict__ rows,
+                                                    const int* __restrict__ cols, int drop_lower, int* row_count,
+                                                    uint32_t* __restrict__ rank, int* flag)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if(t >= n) return;
-    const int r = rows[t], c = cols[t];
-    if(r < 0 || r >= nr || c < 0 || c >= nr)
+    const int lane = threadIdx.x & 63;
+    int  r = -1;
+    bool ok = false;
+    if(t < n)
     {
-        atomicOr(flag, (int)kBadIndex);
-        return;
+        r = rows[t];
+        const int c = cols[t];
+        if(r < 0 || r >= nr || c < 0 || c >= nr)
+            atomicOr(flag, (int)kBadIndex);
+        else
+            ok = !(drop_lower && r > c);
     }
-    if(drop_lower && r > c) return;
-    atomicAdd(&row_count[r], 1);
+    unsigned long long left = __ballot(ok);
+    int leader = lane, before = 0, size = ok ? 1 : 0;
+    for(int k = 0; k < kMerge && left; ++k)
+    {
+        const int first = __ffsll((long long)left) - 1;
+        const int row = __builtin_amdgcn_readlane(r, first);
+        const bool mine = ok && r == row;
+        const unsigned long long same = __ballot(mine);
+        if(mine)
+        {
+            leader = first;
+            before = __popcll(same & ((1ull << lane) - 1ull));
+            size   = __popcll(same);
+        }
+        left &= ~same;
+    }
+    int base = 0;
+    if(ok && leader == lane) base = atomicAdd(&row_count[r], size);
+    base = __shfl(base, leader, 64);
+    if(t < n) rank[t] = ok ? (uint32_t)(base + before) : kNone;
 }
 
-__global__ void __launch_bounds__(256) k_conv_scatter(int n, int nr, const int* rows, const int* cols, int drop_lower,
-                                                      const int* row_start, int* cursor, uint32_t* bucket)
+__global__ void __launch_bounds__(256) k_conv_scatter(int n, const int* __restrict__ rows,
+                                                      const uint32_t* __restrict__ rank,
+                                                      const int* __restrict__ row_start, uint32_t* __restrict__ bucket)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if(t >= n) return;
-    const int r = rows[t], c = cols[t];
-    if(r < 0 || r >= nr || c < 0 || c >= nr) return;
-    if(drop_lower && r > c) return;
-    bucket[row_start[r] + atomicAdd(&cursor[r], 1)] = (uint32_t)t;
+    const uint32_t k = rank[t];
+    if(k != kNone) bucket[row_start[rows[t]] + k] = (uint32_t)t;
 }
 
 // exclusive scan, level 1: each workgroup scans one tile and emits its total
@@ -81,123 +123,204 @@ __global__ void __launch_bounds__(kScanBlock) k_scan_tiles(const int* in, int* o
     if(threadIdx.x == kScanBlock - 1) tile_sums[blockIdx.x] = s[kScanBlock - 1];
 }
 
-// level 2: one workgroup scans the tile totals in place (exclusive), any count
-__global__ void __launch_bounds__(kScanBlock) k_scan_totals(int* tile_sums, int tiles, int* total)
+// level 2: every workgroup sums the totals of the tiles before its own
+__global__ void __launch_bounds__(kScanBlock) k_scan_add(int* out, int m, const int* tile_sums, int tiles)
 {
     __shared__ int s[kScanBlock];
-    int carry = 0;
-    for(int b = 0; b < tiles; b += kScanBlock)
+    const int mine = blockIdx.x;
+    int before = 0;
+    for(int i = threadIdx.x; i < mine; i += kScanBlock) before += tile_sums[i];
+    s[threadIdx.x] = before;
+    __syncthreads();
+    for(int off = kScanBlock / 2; off > 0; off >>= 1)
     {
-        const int i = b + threadIdx.x;
-        const int v = i < tiles ? tile_sums[i] : 0;
-        s[threadIdx.x] = v;
+        if((int)threadIdx.x < off) s[threadIdx.x] += s[threadIdx.x + off];
         __syncthreads();
-        for(int off = 1; off < kScanBlock; off <<= 1)
-        {
-            const int add = threadIdx.x >= off ? s[threadIdx.x - off] : 0;
-            __syncthreads();
-            s[threadIdx.x] += add;
-            __syncthreads();
-        }
-        if(i < tiles) tile_sums[i] = carry + s[threadIdx.x] - v;
-        const int chunk_total = s[kScanBlock - 1];
-        __syncthreads();
-        carry += chunk_total;
     }
-    if(threadIdx.x == 0) *total = carry;
-}
-
-__global__ void __launch_bounds__(kScanBlock) k_scan_add(int* out, int m, const int* tile_sums, const int* total)
-{
-    const int i = blockIdx.x * kScanTile + threadIdx.x;
-    const int add = tile_sums[blockIdx.x];
+    const int add = s[0];
+    const int i = mine * kScanTile + threadIdx.x;
 #pragma unroll
     for(int k = 0; k < kScanItems; ++k)
         if(i + k * kScanBlock < m) out[i + k * kScanBlock] += add;
-    if(blockIdx.x == 0 && threadIdx.x == 0) out[m] = *total;
+    if(mine == tiles - 1 && threadIdx.x == 0) out[m] = add + tile_sums[mine];
 }
 
-// One wavefront per block row: order the row's triplets by (col, input
-// index), mark the first entry of every column run, and record where each
-// unique block's run starts (written into the row's own bucket range).
-__global__ void __launch_bounds__(64) k_conv_row_sort(int nr, const int* row_start, uint32_t* bucket,
-                                                      const int* cols, unsigned long long* gkeys,
-                                                      unsigned long long* gsorted, int* seg, int* uniq)
+// One wavefront per block row of at most kRowRegs triplets: ordered by (col,
+// input index) in registers, each lane ranking its two keys against every
+// other (readlane broadcasts), then the input indices in that order with the
+// first of every column run marked.  Longer rows are listed for the kernel
+// below.
+__global__ void __launch_bounds__(256) k_conv_row_sort(int nr, const int* __restrict__ row_start,
+                                                       uint32_t* __restrict__ bucket, const int* __restrict__ cols,
+                                                       int* __restrict__ uniq, int* __restrict__ long_rows, int* n_long)
 {
-    __shared__ unsigned long long s_keys[kRowCap], s_sorted[kRowCap];
-    const int r = blockIdx.x;
+    const int r = blockIdx.x * 4 + (int)(threadIdx.x >> 6);
     if(r >= nr) return;
-    const int rs = row_start[r], L = row_start[r + 1] - rs;
-    const int lane = threadIdx.x;
-    if(L == 0)
+    const int rs = row_start[r], L = row_start[r + 1] - rs, lane = threadIdx.x & 63;
+    if(L > kRowRegs)
     {
-        if(lane == 0) uniq[r] = 0;
+        if(lane == 0) long_rows[atomicAdd(n_long, 1)] = r;
         return;
     }
-    unsigned long long* keys   = L <= kRowCap ? s_keys : gkeys + rs;
-    unsigned long long* sorted = L <= kRowCap ? s_sorted : gsorted + rs;
-    for(int i = lane; i < L; i += 64)
+    uint32_t t[2], c[2];
+    int      rank[2] = {0, 0};
+#pragma unroll
+    for(int h = 0; h < 2; ++h) t[h] = lane + 64 * h < L ? bucket[rs + lane + 64 * h] : 0u;
+#pragma unroll
+    for(int h = 0; h < 2; ++h) c[h] = lane + 64 * h < L ? (uint32_t)cols[t[h]] : 0xffffffffu;
+    unsigned long long key[2];
+#pragma unroll
+    for(int h = 0; h < 2; ++h) key[h] = ((unsigned long long)c[h] << 32) | t[h];
+    const int n0 = __builtin_amdgcn_readfirstlane(min(L, 64)), n1 = __builtin_amdgcn_readfirstlane(L - min(L, 64));
+    for(int j = 0; j < n0; ++j)
     {
-        const uint32_t t = bucket[rs + i];
-        keys[i] = ((unsigned long long)(uint32_t)cols[t] << 32) | t;
+        const unsigned long long k = ((unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)c[0], j) << 32) |
+                                     (uint32_t)__builtin_amdgcn_readlane((int)t[0], j);
+        rank[0] += k < key[0];
+        rank[1] += k < key[1];
     }
-    __syncthreads();
-    // keys are distinct (the input index is part of the key): rank = position
-    for(int i = lane; i < L; i += 64)
+    for(int j = 0; j < n1; ++j)
     {
-        const unsigned long long k = keys[i];
-        int rank = 0;
-        for(int j = 0; j < L; ++j) rank += keys[j] < k;
-        sorted[rank] = k;
+        const unsigned long long k = ((unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)c[1], j) << 32) |
+                                     (uint32_t)__builtin_amdgcn_readlane((int)t[1], j);
+        rank[0] += k < key[0];
+        rank[1] += k < key[1];
     }
-    __syncthreads();
-    int count = 0;  // unique blocks before this 64-entry slice
-    for(int base = 0; base < L; base += 64)
-    {
-        const int i = base + lane;
-        bool head = false;
-        unsigned long long k = 0;
-        if(i < L)
+    // to sorted order through LDS (keys are distinct: rank = position)
+    __shared__ uint32_t s_t[4][kRowRegs], s_c[4][kRowRegs];
+    uint32_t* st = s_t[threadIdx.x >> 6];
+    uint32_t* sc = s_c[threadIdx.x >> 6];
+#pragma unroll
+    for(int h = 0; h < 2; ++h)
+        if(lane + 64 * h < L)
         {
-            k = sorted[i];
-            head = i == 0 || (k >> 32) != (sorted[i - 1] >> 32);
+            st[rank[h]] = t[h];
+            sc[rank[h]] = c[h];
         }
-        const unsigned long long heads = __ballot(head);
-        const int before = __popcll(heads & ((1ull << lane) - 1ull));
-        if(head) seg[rs + count + before] = rs + i;
-        count += __popcll(heads);
-        __syncthreads();  // every lane has read sorted[] of this slice before bucket[] is overwritten
-        if(i < L) bucket[rs + i] = (uint32_t)(k & 0xffffffffu);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    int count = 0;
+#pragma unroll
+    for(int h = 0; h < 2; ++h)
+    {
+        const int  i = lane + 64 * h;
+        const bool head = i < L && (i == 0 || sc[i] != sc[i - 1]);
+        if(i < L) bucket[rs + i] = st[i] | (head ? kHead : 0u);
+        count += __popcll(__ballot(head));
     }
     if(lane == 0) uniq[r] = count;
 }
 
-// One wavefront per block row: sum every run (input order) into its unique block.
-__global__ void __launch_bounds__(64) k_conv_write(int nr, const int* row_start, const uint32_t* bucket,
-                                                   const int* seg, const int* uniq, const int* out_start,
-                                                   const int* cols, const double* vals, int* out_rows,
-                                                   int* out_cols, double* out_vals)
+// The rows longer than kRowRegs, one wavefront each, with the keys in LDS (or
+// global scratch past kRowCap).
+__global__ void __launch_bounds__(64) k_conv_row_sort_long(const int* __restrict__ long_rows, const int* n_long,
+                                                           const int* __restrict__ row_start, uint32_t* bucket,
+                                                           const int* __restrict__ cols, unsigned long long* gkeys,
+                                                           unsigned long long* gsorted, int* uniq)
 {
-    const int r = blockIdx.x;
-    if(r >= nr) return;
-    const int rs = row_start[r], re = row_start[r + 1], U = uniq[r], o0 = out_start[r];
-    for(int u = threadIdx.x; u < U; u += 64)
+    __shared__ unsigned long long s_keys[kRowCap], s_sorted[kRowCap];
+    const int lane = threadIdx.x, rows_left = *n_long;
+    for(int q = blockIdx.x; q < rows_left; q += gridDim.x)
     {
-        const int s0 = seg[rs + u], s1 = u + 1 < U ? seg[rs + u + 1] : re;
-        double acc[9];
-#pragma unroll
-        for(int c = 0; c < 9; ++c) acc[c] = 0.0;
-        for(int k = s0; k < s1; ++k)
+        const int r = long_rows[q], rs = row_start[r], L = row_start[r + 1] - rs;
+        unsigned long long* keys   = L <= kRowCap ? s_keys : gkeys + rs;
+        unsigned long long* sorted = L <= kRowCap ? s_sorted : gsorted + rs;
+        for(int i = lane; i < L; i += 64)
         {
-            const double* B = vals + 9 * (long long)bucket[k];
-#pragma unroll
-            for(int c = 0; c < 9; ++c) acc[c] += B[c];
+            const uint32_t t = bucket[rs + i];
+            keys[i] = ((unsigned long long)(uint32_t)cols[t] << 32) | t;
         }
-        const long long o = o0 + u;
-        out_rows[o] = r;
-        out_cols[o] = cols[bucket[s0]];
+        __syncthreads();
+        // keys are distinct (the input index is part of the key): rank = position
+        for(int i = lane; i < L; i += 64)
+        {
+            const unsigned long long k = keys[i];
+            int rank = 0;
+            for(int j = 0; j < L; ++j) rank += keys[j] < k;
+            sorted[rank] = k;
+        }
+        __syncthreads();
+        int count = 0;
+        for(int base = 0; base < L; base += 64)
+        {
+            const int i = base + lane;
+            const unsigned long long k = i < L ? sorted[i] : 0;
+            const bool head = i < L && (i == 0 || (k >> 32) != (sorted[i - 1] >> 32));
+            count += __popcll(__ballot(head));
+            if(i < L) bucket[rs + i] = (uint32_t)(k & 0xffffffffu) | (head ? kHead : 0u);
+        }
+        if(lane == 0) uniq[r] = count;
+        __syncthreads();  // the next row reuses the LDS
+    }
+}
+
+// One wavefront per block row: its triplets' values pass through LDS in
+// chunks of 63 (nine lanes read a block's 72 contiguous bytes), and the lanes
+// sum the runs there, in input order, into 9 contiguous values per unique
+// block.  A run that a chunk cuts is carried over to the next.
+constexpr int kWriteChunk = 63;
+__global__ void __launch_bounds__(256) k_conv_write(int nr, const int* __restrict__ row_start,
+                                                    const uint32_t* __restrict__ bucket,
+                                                    const int* __restrict__ out_start, const int* __restrict__ cols,
+                                                    const double* __restrict__ vals, int* __restrict__ out_rows,
+                                                    int* __restrict__ out_cols, double* __restrict__ out_vals)
+{
+    __shared__ double s_v[4][kWriteChunk * 9];
+    __shared__ double s_carry[4][2][9];  // read from one, written to the other
+    __shared__ int    s_head[4][64];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = blockIdx.x * 4 + wave;
+    if(r >= nr) return;
+    const int rs = __builtin_amdgcn_readfirstlane(row_start[r]);
+    const int re = __builtin_amdgcn_readfirstlane(row_start[r + 1]);
+    long long o = out_start[r];  // unique blocks finished before the current chunk's first run
+    double* V = s_v[wave];
+    int     flip = 0;
+    int*    H = s_head[wave];
+    const int g = lane / 9, q = lane % 9;
+    for(int c0 = rs; c0 < re; c0 += kWriteChunk)
+    {
+        const int n = min(kWriteChunk, re - c0);
+        const uint32_t code = lane < n ? bucket[c0 + lane] : 0u;
+        const int t = (int)(code & ~kHead);
+        const unsigned long long heads = __ballot(lane < n && (code & kHead));
+        const int cont = heads & 1ull ? 0 : 1;  // the chunk begins inside a run
+        const int runs = __popcll(heads) + cont;
+        const bool open = c0 + n < re && !(bucket[c0 + n] & kHead);  // its last run goes on
+        if(lane < n && (code & kHead))
+        {
+            const int k = __popcll(heads & ((1ull << lane) - 1ull)) + cont;
+            H[k] = lane;
+            out_rows[o + k] = r;
+            out_cols[o + k] = cols[t];
+        }
+        if(cont && lane == 0) H[0] = 0;
+        double v[9];
 #pragma unroll
-        for(int c = 0; c < 9; ++c) out_vals[9 * o + c] = acc[c];
+        for(int k = 0; k < 9; ++k)
+        {
+            const int e = min(g + 7 * k, n - 1);
+            v[k] = __builtin_nontemporal_load(vals + 9 * (long long)__shfl(t, e, 64) + q);
+        }
+#pragma unroll
+        for(int k = 0; k < 9; ++k)
+            if(g + 7 * k < n && lane < 63) V[9 * (g + 7 * k) + q] = v[k];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        for(int i = lane; i < 9 * runs; i += 64)
+        {
+            const int k = i / 9, c = i - 9 * k;
+            const int b = H[k], e = k + 1 < runs ? H[k + 1] : n;
+            double acc = k == 0 && cont ? s_carry[wave][flip][c] : 0.0;
+            for(int j = b; j < e; ++j) acc += V[9 * j + c];
+            if(k + 1 == runs && open)
+                s_carry[wave][flip ^ 1][c] = acc;
+            else
+                out_vals[9 * o + i] = acc;
+        }
+        o += runs - (open ? 1 : 0);
+        flip ^= 1;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
     }
 }
 
@@ -223,8 +346,8 @@ void grow(T*& p, size_t& cap, size_t need)
 
 Converter::~Converter()
 {
-    for(void* p : {(void*)row_count_, (void*)row_start_, (void*)cursor_, (void*)bucket_, (void*)seg_, (void*)uniq_,
-                   (void*)out_start_, (void*)tiles_, (void*)flag_, (void*)keys_, (void*)sorted_})
+    for(void* p : {(void*)row_count_, (void*)row_start_, (void*)rank_, (void*)bucket_, (void*)uniq_, (void*)out_start_,
+                   (void*)tiles_, (void*)long_rows_, (void*)keys_, (void*)sorted_})
         if(p) (void)hipFree(p);
     if(h_pinned_) (void)hipHostFree(h_pinned_);
 }
@@ -233,10 +356,9 @@ void Converter::scan(const int* in, int* out, int m, hipStream_t st)
 {
     // out[0..m] = exclusive prefix sums of in[0..m-1]; out[m] = total
     const int tiles = std::max(1, (m + kScanTile - 1) / kScanTile);
-    grow(tiles_, tiles_cap_, (size_t)tiles + 1);
+    grow(tiles_, tiles_cap_, (size_t)tiles);
     hipLaunchKernelGGL(k_scan_tiles, dim3(tiles), dim3(kScanBlock), 0, st, in, out, m, tiles_);
-    hipLaunchKernelGGL(k_scan_totals, dim3(1), dim3(kScanBlock), 0, st, tiles_, tiles, tiles_ + tiles);
-    hipLaunchKernelGGL(k_scan_add, dim3(tiles), dim3(kScanBlock), 0, st, out, m, tiles_, tiles_ + tiles);
+    hipLaunchKernelGGL(k_scan_add, dim3(tiles), dim3(kScanBlock), 0, st, out, m, tiles_, tiles);
     CONV_HIP(hipGetLastError());
 }
 
@@ -247,36 +369,36 @@ int Converter::convert(int n, int n_block_rows, const int* rows, const int* cols
     if(n == 0) return 0;
     if(!rows || !cols || !vals || !out_rows || !out_cols || !out_vals) throw std::invalid_argument("null pointer");
     const int nr = n_block_rows;
-    grow(row_count_, row_count_cap_, (size_t)nr);
+    // row counts, then the bad-index flag and the count of long rows (one clear)
+    grow(row_count_, row_count_cap_, (size_t)nr + 2);
     grow(row_start_, row_start_cap_, (size_t)nr + 1);
-    grow(cursor_, cursor_cap_, (size_t)nr);
     grow(uniq_, uniq_cap_, (size_t)nr);
     grow(out_start_, out_start_cap_, (size_t)nr + 1);
+    grow(long_rows_, long_rows_cap_, (size_t)nr);
+    grow(rank_, rank_cap_, (size_t)n);
     grow(bucket_, bucket_cap_, (size_t)n);
-    grow(seg_, seg_cap_, (size_t)n);
     grow(keys_, keys_cap_, (size_t)n);
     grow(sorted_, sorted_cap_, (size_t)n);
-    grow(flag_, flag_cap_, 1);
     if(!h_pinned_) CONV_HIP(hipHostMalloc((void**)&h_pinned_, 2 * sizeof(int), hipHostMallocDefault));
+    int *flag = row_count_ + nr, *n_long = flag + 1;
 
-    CONV_HIP(hipMemsetAsync(row_count_, 0, sizeof(int) * nr, st));
-    CONV_HIP(hipMemsetAsync(cursor_, 0, sizeof(int) * nr, st));
-    CONV_HIP(hipMemsetAsync(flag_, 0, sizeof(int), st));
+    CONV_HIP(hipMemsetAsync(row_count_, 0, sizeof(int) * ((size_t)nr + 2), st));
     hipLaunchKernelGGL(k_conv_count, dim3(grid_for(n, 256)), dim3(256), 0, st, n, nr, rows, cols, drop_lower,
-                       row_count_, flag_);
+                       row_count_, rank_, flag);
     CONV_HIP(hipGetLastError());
     scan(row_count_, row_start_, nr, st);
-    hipLaunchKernelGGL(k_conv_scatter, dim3(grid_for(n, 256)), dim3(256), 0, st, n, nr, rows, cols, drop_lower,
-                       row_start_, cursor_, bucket_);
-    hipLaunchKernelGGL(k_conv_row_sort, dim3(nr), dim3(64), 0, st, nr, row_start_, bucket_, cols, keys_, sorted_,
-                       seg_, uniq_);
+    hipLaunchKernelGGL(k_conv_scatter, dim3(grid_for(n, 256)), dim3(256), 0, st, n, rows, rank_, row_start_, bucket_);
+    hipLaunchKernelGGL(k_conv_row_sort, dim3(grid_for(nr, 4)), dim3(256), 0, st, nr, row_start_, bucket_, cols, uniq_,
+                       long_rows_, n_long);
+    hipLaunchKernelGGL(k_conv_row_sort_long, dim3((unsigned)std::min(nr, kLongGrid)), dim3(64), 0, st, long_rows_,
+                       n_long, row_start_, bucket_, cols, keys_, sorted_, uniq_);
     CONV_HIP(hipGetLastError());
     scan(uniq_, out_start_, nr, st);
-    hipLaunchKernelGGL(k_conv_write, dim3(nr), dim3(64), 0, st, nr, row_start_, bucket_, seg_, uniq_, out_start_, cols,
+    hipLaunchKernelGGL(k_conv_write, dim3(grid_for(nr, 4)), dim3(256), 0, st, nr, row_start_, bucket_, out_start_, cols,
                        vals, out_rows, out_cols, out_vals);
     CONV_HIP(hipGetLastError());
     CONV_HIP(hipMemcpyAsync(h_pinned_, out_start_ + nr, sizeof(int), hipMemcpyDeviceToHost, st));
-    CONV_HIP(hipMemcpyAsync(h_pinned_ + 1, flag_, sizeof(int), hipMemcpyDeviceToHost, st));
+    CONV_HIP(hipMemcpyAsync(h_pinned_ + 1, flag, sizeof(int), hipMemcpyDeviceToHost, st));
     CONV_HIP(hipStreamSynchronize(st));
     if(h_pinned_[1] & kBadIndex) throw std::invalid_argument("triplet block index outside [0, n_block_rows)");
     return h_pinned_[0];

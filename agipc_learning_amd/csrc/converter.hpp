@@ -25,19 +25,18 @@ class Converter
   private:
     void scan(const int* in, int* out, int m, hipStream_t st);
 
-    int*                row_count_ = nullptr;
+    int*                row_count_ = nullptr;  // per row; then the bad-index flag and the long rows' count
     int*                row_start_ = nullptr;
-    int*                cursor_    = nullptr;
+    uint32_t*           rank_      = nullptr;  // per triplet: its place in its row's bucket
     uint32_t*           bucket_    = nullptr;
-    int*                seg_       = nullptr;
     int*                uniq_      = nullptr;
     int*                out_start_ = nullptr;
     int*                tiles_     = nullptr;
-    int*                flag_      = nullptr;
+    int*                long_rows_ = nullptr;
     unsigned long long* keys_      = nullptr;
     unsigned long long* sorted_    = nullptr;
-    size_t row_count_cap_ = 0, row_start_cap_ = 0, cursor_cap_ = 0, bucket_cap_ = 0, seg_cap_ = 0, uniq_cap_ = 0,
-           out_start_cap_ = 0, tiles_cap_ = 0, flag_cap_ = 0, keys_cap_ = 0, sorted_cap_ = 0;
+    size_t row_count_cap_ = 0, row_start_cap_ = 0, rank_cap_ = 0, bucket_cap_ = 0, uniq_cap_ = 0, out_start_cap_ = 0,
+           tiles_cap_ = 0, long_rows_cap_ = 0, keys_cap_ = 0, sorted_cap_ = 0;
     int* h_pinned_ = nullptr;
 };
 }  // namespace masx

@@ -56,8 +56,8 @@ def test_spmv64_row_tiles_and_chunks(oracle, n, per_row, hub):
 
 @pytest.mark.parametrize("n_tets", [1, 63, 64, 65, 190])
 def test_fem_assemble_tet_groups_and_chunks(oracle, n_tets):
-    """Assembly around the 64-tet groups and 64-target tiles, and a tile whose
-    contributions exceed a 504-entry chunk (every tet shares two vertices).
+    """Assembly around the 64-tet groups and 32-target tiles, and a tile whose
+    contributions exceed a 252-entry chunk (every tet shares two vertices).
     Bound as in the other assembly tests (two routes of the same 64-bit
     projection, 1e-11 of the largest value)."""
     from agipc_learning_amd import adjoint
@@ -79,3 +79,23 @@ def test_fem_assemble_tet_groups_and_chunks(oracle, n_tets):
     want = np.stack([A[3 * r:3 * r + 3, 3 * c:3 * c + 3].reshape(9, order="F") for r, c in zip(rows, cols)])
     assert np.abs(plain - want).max() <= 1e-11 * np.abs(want).max()
     assert np.abs(got - base - want).max() <= 1e-11 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("lengths,spread", [([1], 1), ([62, 63, 64, 65], 40), ([126, 127, 128, 129, 130], 9),
+                                            ([63, 126, 189, 64, 0, 0, 70], 1), ([1024, 1025, 3, 1100], 7),
+                                            ([90] * 70 + [0] * 3, 25)])
+def test_converter_row_lengths(oracle, lengths, spread):
+    """Rows around the register sort (64 and 128 triplets), the LDS sort (1,024)
+    and the 63-triplet chunks of the sums, with runs that chunks cut; bit for
+    bit as the oracle (sums in input order)."""
+    rng = np.random.default_rng(len(lengths) + spread)
+    r = np.repeat(np.arange(len(lengths)), lengths).astype(np.int32)
+    r = rng.permutation(r).astype(np.int32)
+    c = rng.integers(0, min(spread, len(lengths)), len(r)).astype(np.int32)
+    v = rng.standard_normal((len(r), 9))
+    conv = native.Converter()
+    for drop_lower in (False, True):
+        got = conv.convert(dev(r), dev(c), dev(v), len(lengths), drop_lower)
+        want = oracle.convert_triplets(r, c, v, drop_lower)
+        for a, b in zip(got, want):
+            assert np.array_equal(host(a), b)
