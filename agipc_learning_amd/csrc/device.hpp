@@ -56,7 +56,8 @@ struct DevData
 {
     // sizes
     int n_rows, n_sys, bank, n_banks, n_fine_banks;
-    int mas_waves;                      // waves per workgroup of the FP32 MAS local kernel (4 or 8)
+    int mas_waves;                      // MAS local variant: 2 lane tiles, 1 MFMA, 4 / 8 waves, 5 / 9 staged
+    int mas_nt;                         // 1: the lane-tile kernel reads the inverses with nontemporal loads
     int spmv_nt;                        // 1: the SpMV reads the matrix with nontemporal loads
     int spmv_bodies;                    // 1: the SpMV layout has tiles of affine bodies
     int factor_waves;                   // waves per bank of the MAS factor (1 or 2)
@@ -94,6 +95,7 @@ struct DevData
     const float*    minv_scale;  // per bank (half-precision storage is scaled to [-1, 1])
     const int*      bank_vec;
     const int*      bank_sys;
+    const int*      bank_live;   // per coarse bank: its nodes that exist
     const int*      bank_kind;   // 0 level 0, 1 level 1, 2 level >= 2
     const int*      comp_ptr;
     const uint32_t* comp_mask;

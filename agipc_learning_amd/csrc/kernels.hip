@@ -15,6 +15,7 @@
 //  * kernels of a finished system return at once, so a captured chunk of
 //    iterations can run past convergence at negligible cost.
 #include "kernels.hpp"
+#include "lane_tiles.hpp"
 #include "mas_tiles.hpp"
 #include "spmv_layout.hpp"
 
@@ -22,6 +23,7 @@
 #include <hip/hip_ext.h>
 #include <hip/hip_fp16.h>
 
+#include <algorithm>
 #include <type_traits>
 
 namespace masx
@@ -150,7 +152,7 @@ __device__ __forceinline__ uint32_t lane_xor16(uint32_t x, uint32_t& other)
     other = r[1];
     return r[0];
 }
-constexpr int kDppRor8 = 0x128, kDppRor4 = 0x124, kDppXor2 = 0x4e, kDppXor1 = 0xb1;
+constexpr int kDppRor8 = 0x128, kDppRor4 = 0x124, kDppXor2 = 0x4e, kDppXor1 = 0xb1, kDppHalfMirror = 0x141;
 template <int CTRL>
 __device__ __forceinline__ float dpp_move(float v)
 {
@@ -287,6 +289,13 @@ __device__ __forceinline__ int xcd_tile(int bid, int n)
     return xcd * per + (xcd < rem ? xcd : rem) + k;
 }
 
+// LDS written by the wave's lanes is readable by all of them after this
+__device__ __forceinline__ void wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 __device__ __forceinline__ bool finite_d(double v) { return isfinite(v); }
 
 }  // namespace
@@ -414,21 +423,36 @@ __global__ void __launch_bounds__(256) k_gal_gather(const double* fine, double* 
 // 16-bit halves of 5 words per block (the tenth half is zero).
 // Half-precision inverses of 32-slot banks are stored as MFMA tiles (the
 // tile layout of mas_tiles.hpp) when the MFMA local kernel reads them
-// (DevData::mas_waves == 1); otherwise, and for 16-slot banks and FP32, by
-// block diagonals.
+// (DevData::mas_waves == 1), every inverse as lane tiles when k_mas_lanes does
+// (mas_waves == 2), otherwise by block diagonals.
 template <int BANK, typename T>
 constexpr bool kTileCapable = BANK == 32 && !std::is_same<T, float>::value;
 
+enum InverseLayout : int { kByDiagonals = 0, kMfmaTiles = 1, kLaneTiles = 2 };
+
 template <int BANK, typename T>
-__device__ __forceinline__ int inverse_slots(int i, int j, bool tiles, int (&slot)[2])
+__device__ __forceinline__ int inverse_layout(int mas_waves)
 {
+    return mas_waves == 2 ? kLaneTiles : kTileCapable<BANK, T> && mas_waves == 1 ? kMfmaTiles : kByDiagonals;
+}
+
+template <int BANK, typename T>
+__device__ __forceinline__ int inverse_slots(int i, int j, int layout, int (&slot)[2])
+{
+    if(layout == kLaneTiles)
+    {
+        slot[0] = lane_tile_slot(BANK, sizeof(T) == 4, i, j);
+        if(i == j || i / 8 != j / 8) return 1;
+        slot[1] = lane_tile_slot(BANK, sizeof(T) == 4, j, i);  // a diagonal tile is stored whole
+        return 2;
+    }
     // Stored positions of element (i, j), i >= j, of a bank's inverse,
     // bank-relative, in units of the stored value (an FP32 float, or a
     // 16-bit half of the half-precision layouts): one, or two where the
     // element has a mirror in the same diagonal block or tile.
     if constexpr(kTileCapable<BANK, T>)
     {
-        if(tiles)
+        if(layout == kMfmaTiles)
         {
             // (i, j) is the upper element (j, i); a diagonal tile also takes its mirror (i, j)
             slot[0] = tile_half_index(j, i);
@@ -456,15 +480,16 @@ __device__ __forceinline__ int inverse_slots(int i, int j, bool tiles, int (&slo
     return nc;
 }
 
-// Bytes of one bank's stored inverse (the MFMA tile layout, the half
+// Bytes of one bank's stored inverse (the MFMA or lane tiles, the half
 // block-diagonal layout of five words per block, or FP32 nine floats per
 // block); every position is either an element's (inverse_slots) or a zero.
 template <int BANK, typename T>
-__device__ __forceinline__ int bank_inverse_bytes(bool tiles)
+__device__ __forceinline__ int bank_inverse_bytes(int layout)
 {
     constexpr int NBLK = BANK * (BANK + 1) / 2;
+    if(layout == kLaneTiles) return lane_tile_values(BANK, sizeof(T) == 4) * (int)sizeof(T);
     if constexpr(kTileCapable<BANK, T>)
-        if(tiles) return kTileBankHalves * 2;
+        if(layout == kMfmaTiles) return kTileBankHalves * 2;
     return std::is_same<T, float>::value ? NBLK * 9 * 4 : NBLK * 5 * 4;
 }
 
@@ -475,9 +500,9 @@ __device__ __forceinline__ int bank_inverse_bytes(bool tiles)
 // it into the stored layout, written in 16-byte stores.
 template <int BANK, typename T>
 __device__ __forceinline__ void write_bank_inverse(const float* L, const unsigned short* __restrict__ map, void* out,
-                                                   int bank, bool tiles)
+                                                   int bank, int layout)
 {
-    const int n16 = bank_inverse_bytes<BANK, T>(tiles) / 16;
+    const int n16 = bank_inverse_bytes<BANK, T>(layout) / 16;
     auto val = [&](unsigned short e) { return e != 0xffffu ? L[e] : 0.f; };
     if constexpr(std::is_same<T, float>::value)
     {
@@ -513,7 +538,7 @@ __device__ __forceinline__ void write_bank_inverse(const float* L, const unsigne
 // keeps there (the map was filled with 0xffff: positions no element takes
 // hold zero).  One thread per element.
 template <int BANK, typename T>
-__global__ void __launch_bounds__(256) k_inverse_map(unsigned short* map, int tiles)
+__global__ void __launch_bounds__(256) k_inverse_map(unsigned short* map, int layout)
 {
     constexpr int DIM = 3 * BANK, NE = DIM * (DIM + 1) / 2;
     static_assert(NE < 0xffff, "element indices fit 16 bits");
@@ -523,7 +548,7 @@ __global__ void __launch_bounds__(256) k_inverse_map(unsigned short* map, int ti
     while((i + 1) * (i + 2) / 2 <= e) ++i;
     const int j = e - i * (i + 1) / 2;
     int slot[2];
-    const int n = inverse_slots<BANK, T>(i, j, tiles != 0, slot);
+    const int n = inverse_slots<BANK, T>(i, j, layout, slot);
     for(int u = 0; u < n; ++u) map[slot[u]] = (unsigned short)e;
 }
 
@@ -643,7 +668,7 @@ __global__ void __launch_bounds__(128) k_mas_factor_sym(DevData d, const double*
     constexpr int NH    = factor_pass_max(DIM, NPASS);
     constexpr int NS    = NH > 2 * DIM + 4 ? NH : 2 * DIM + 4;
     constexpr bool kHalf = !std::is_same<T, float>::value;
-    const bool tiles = kTileCapable<BANK, T> && d.mas_waves == 1;  // the MFMA local kernel's layout
+    const int layout = inverse_layout<BANK, T>(d.mas_waves);
     static_assert(DIM % 16 == 0, "the 8 x 16 grid must tile the bank matrix");
     __shared__ __align__(16) double S[NS];
     __shared__ double red[2];
@@ -789,7 +814,7 @@ __global__ void __launch_bounds__(128) k_mas_factor_sym(DevData d, const double*
             if(i >= j) Lf[i * (i + 1) / 2 + j] = (float)(kHalf ? v * inv_scale : v);
         }
     __syncthreads();
-    write_bank_inverse<BANK, T>(Lf, d.inv_map, out, bank, tiles);
+    write_bank_inverse<BANK, T>(Lf, d.inv_map, out, bank, layout);
     if(tid == 0 && bad && status) atomicAdd(status, bad);
 }
 
@@ -822,7 +847,7 @@ __global__ void __launch_bounds__(64) k_mas_factor_wave(DevData d, const double*
     constexpr int NH    = factor_pass_max(DIM, NPASS);
     constexpr int NS    = NH > 2 * DIM ? NH : 2 * DIM;
     constexpr bool kHalf = !std::is_same<T, float>::value;
-    const bool tiles = kTileCapable<BANK, T> && d.mas_waves == 1;  // the MFMA local kernel's layout
+    const int layout = inverse_layout<BANK, T>(d.mas_waves);
     static_assert(DIM % 8 == 0, "the 8 x 8 grid must tile the bank matrix");
     __shared__ __align__(16) double S[NS];
     double* H  = S;
@@ -958,7 +983,7 @@ __global__ void __launch_bounds__(64) k_mas_factor_wave(DevData d, const double*
             if(i >= j) Lf[i * (i + 1) / 2 + j] = (float)(kHalf ? v * inv_scale : v);
         }
     __syncthreads();
-    write_bank_inverse<BANK, T>(Lf, d.inv_map, out, bank, tiles);
+    write_bank_inverse<BANK, T>(Lf, d.inv_map, out, bank, layout);
     if(tid == 0 && bad && status) atomicAdd(status, bad);
 }
 
@@ -1450,6 +1475,226 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4,
         float* dst = (pick(s_kind, lb) == 0 ? d.z : d.Zc) + 3 * (long long)(pick(s_vec, lb) + I);
         dst[0] = z0; dst[1] = z1; dst[2] = z2;
     }
+}
+
+// ---- MAS local solve on lane tiles -----------------------------------------
+// One wave per bank.  The dim x dim inverse (dim = 3 BANK) is cut into 8 x 8
+// tiles over an 8 x 8 grid of lanes: lane (ty, tx) holds element
+// (ty + 8 a, tx + 8 b) of every stored tile a >= b, 78 values of a 32-slot
+// bank in registers, and multiplies each by r of its column and, off the
+// diagonal tiles, by r of its row.  That is 144 FMAs and 20 loads of 16 bytes
+// per lane for a whole bank, where the block-diagonal kernels (k_mas_local)
+// spend ~1,450 wave instructions per bank on 4-byte loads, shuffles of every
+// transposed product and index arithmetic: on a few thousand banks those were
+// bound by VALU issue, not by their bytes.  The layout holds 5 % more than the
+// FP32 block diagonals (19,968 B: diagonal tiles are whole) and 7 % less than
+// the MFMA tiles (9,984 B), and measured on 91,066 banks: FP32 296 us (staged
+// block diagonals 291-316), FP16 156 and BF16 150 (MFMA 190), so every size
+// runs it; one 40^3 system's 2,270 banks 9.8 us (four waves 10.4).  The row sums meet over tx and
+// the column sums over ty by exchanges that halve the values each lane keeps
+// (DPP and permlane swaps), and meet each other in LDS.
+// Residuals of level >= 2 banks are sums of their nodes' update-group
+// partials, the lanes split evenly over the live nodes.  Coarse banks (the
+// end of the list) come first, so their longer gathers overlap the others.
+// NT: nontemporal loads, for inverses far larger than the caches.
+template <int BANK>
+struct LaneGrid
+{
+    static constexpr int T = 3 * BANK / 8, NS = T * (T + 1) / 2;  // tiles per row; stored tiles
+};
+
+template <bool NT, typename V>
+__device__ __forceinline__ V ld_inverse(const V* p)
+{
+    if constexpr(NT)
+        return ld_nt(p);
+    else
+        return *p;
+}
+
+// A lane's values of its bank as stored: 16-byte groups of every lane, then
+// the rest of a few values per lane.
+template <int BANK, typename T, bool NT>
+__device__ __forceinline__ void load_lane_tiles(const void* minv, int bank, int lane,
+                                                uint32_t (&raw)[lane_tile_words(BANK, sizeof(T) == 4)])
+{
+    constexpr bool F32 = sizeof(T) == 4;
+    constexpr int W = lane_tile_words(BANK, F32), Q = W / 4, REM = W % 4;
+    const char* base = reinterpret_cast<const char*>(minv) + (size_t)bank * (lane_tile_values(BANK, F32) * sizeof(T));
+#pragma unroll
+    for(int q = 0; q < Q; ++q)
+    {
+        const uint4 v = ld_inverse<NT>(reinterpret_cast<const uint4*>(base) + 64 * q + lane);
+        raw[4 * q] = v.x; raw[4 * q + 1] = v.y; raw[4 * q + 2] = v.z; raw[4 * q + 3] = v.w;
+    }
+    const uint32_t* rest = reinterpret_cast<const uint32_t*>(base) + 256 * Q + REM * lane;
+#pragma unroll
+    for(int q = 0; q < REM; ++q) raw[4 * Q + q] = ld_inverse<NT>(rest + q);
+}
+
+template <typename T, int W>
+__device__ __forceinline__ float lane_tile_value(const uint32_t (&raw)[W], int s)
+{
+    if constexpr(sizeof(T) == 4)
+        return __uint_as_float(raw[s]);
+    else
+        return s & 1 ? hi_half(raw[s / 2], (T*)nullptr) : lo_half(raw[s / 2], (T*)nullptr);
+}
+
+// z = (stored inverse) R over the bank's dim values; R and Y: dim floats of the
+// wave's LDS each.  Afterwards lanes with `mine` hold z[at[k]] in y[k].
+template <int BANK, typename T, int W>
+__device__ __forceinline__ void lane_tile_product(const uint32_t (&raw)[W], const float* R, float* Y, int lane,
+                                                  float (&y)[3], int (&at)[3], bool& mine)
+{
+    constexpr int TT = LaneGrid<BANK>::T, H = TT / 2;
+    static_assert(TT == 12 || TT == 6, "32- or 16-slot banks");
+    const int ty = lane >> 3, tx = lane & 7;
+    float rr[TT], rc[TT], yr[TT], yc[TT];
+#pragma unroll
+    for(int a = 0; a < TT; ++a)
+    {
+        rr[a] = R[ty + 8 * a];
+        rc[a] = R[tx + 8 * a];
+        yr[a] = yc[a] = 0.f;
+    }
+#pragma unroll
+    for(int a = 0; a < TT; ++a)
+#pragma unroll
+        for(int b = 0; b <= a; ++b)
+        {
+            const float v = lane_tile_value<T>(raw, a * (a + 1) / 2 + b);
+            yr[a] += v * rc[b];
+            if(b < a) yc[b] += v * rr[a];
+        }
+    // rows: over tx.  Lanes tx >= 4 keep the upper half of the values, their
+    // mirrors 7 - tx the lower; then (12 rows) tx & 2 keeps three of six
+    float u[H];
+    const bool up = tx >= 4;
+#pragma unroll
+    for(int k = 0; k < H; ++k)
+        u[k] = (up ? yr[k + H] : yr[k]) + dpp_move<kDppHalfMirror>(up ? yr[k] : yr[k + H]);
+    float p[3];
+    int   first = up ? H : 0;
+    if constexpr(TT == 12)
+    {
+        const bool second = tx & 2;
+#pragma unroll
+        for(int k = 0; k < 3; ++k) p[k] = (second ? u[k + 3] : u[k]) + dpp_move<kDppXor2>(second ? u[k] : u[k + 3]);
+        first += second ? 3 : 0;
+    }
+    else
+    {
+#pragma unroll
+        for(int k = 0; k < 3; ++k) p[k] = u[k] + dpp_move<kDppXor2>(u[k]);
+    }
+#pragma unroll
+    for(int k = 0; k < 3; ++k) p[k] += dpp_move<kDppXor1>(p[k]);
+    if((tx & (TT == 12 ? 1 : 3)) == 0)
+#pragma unroll
+        for(int k = 0; k < 3; ++k) Y[ty + 8 * (first + k)] = p[k];
+    // columns: over ty.  A swap of the halves (rows) of two registers and one
+    // add leave one value's sum in the lower, the other's in the upper half
+    float c[H];
+#pragma unroll
+    for(int k = 0; k < H; ++k)
+    {
+        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(yc[k]), __float_as_uint(yc[k + H]), false, false);
+        c[k] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    }
+    int col = lane >= 32 ? H : 0;
+#pragma unroll
+    for(int k = 0; k < 3; ++k)
+    {
+        if constexpr(TT == 12)
+        {
+            const auto r =
+                __builtin_amdgcn_permlane16_swap(__float_as_uint(c[k]), __float_as_uint(c[k + 3]), false, false);
+            y[k] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+        }
+        else
+        {
+            uint32_t o;
+            const uint32_t m = lane_xor16(__float_as_uint(c[k]), o);
+            y[k] = __uint_as_float(m) + __uint_as_float(o);
+        }
+        y[k] += dpp_move<kDppRor8>(y[k]);
+    }
+    if constexpr(TT == 12) col += lane & 16 ? 3 : 0;
+    mine = (lane & (TT == 12 ? 8 : 24)) == 0;
+    wave_sync();
+#pragma unroll
+    for(int k = 0; k < 3; ++k)
+    {
+        at[k] = tx + 8 * (col + k);
+        y[k] += Y[at[k]];
+    }
+}
+
+// Residual of one bank (dim values) into the wave's LDS.
+template <int BANK>
+__device__ __forceinline__ void lane_bank_residual(const DevData& d, int bank, int kind, int vec, int lane, float* R)
+{
+    if(kind < 2)
+    {
+        const float* r = (kind == 0 ? d.r : d.Rc) + 3 * (long long)vec;
+#pragma unroll
+        for(int i = 0; i < 3 * BANK; i += 64)
+            if(i + lane < 3 * BANK) R[i + lane] = r[i + lane];
+        return;
+    }
+    const int m = d.bank_live[bank - d.n_fine_banks];
+    int P = 64;  // lanes per live node: a power of two
+    while(P * m > 64) P >>= 1;
+    const int node = lane / P, sub = lane % P;
+    float a0 = 0.f, a1 = 0.f, a2 = 0.f;
+    if(node < m)
+    {
+        const int end = d.deep_ptr[vec + node + 1];
+#pragma unroll 4
+        for(int k = d.deep_ptr[vec + node] + sub; k < end; k += P)
+        {
+            const long long c = 3 * (long long)d.deep_list[k];
+            a0 += d.part_deep[c]; a1 += d.part_deep[c + 1]; a2 += d.part_deep[c + 2];
+        }
+    }
+    for(int off = P >> 1; off > 0; off >>= 1)
+    {
+        a0 += __shfl_xor(a0, off, 64);
+        a1 += __shfl_xor(a1, off, 64);
+        a2 += __shfl_xor(a2, off, 64);
+    }
+    for(int i = 3 * m + lane; i < 3 * BANK; i += 64) R[i] = 0.f;
+    if(sub == 0 && node < m)
+    {
+        R[3 * node] = a0; R[3 * node + 1] = a1; R[3 * node + 2] = a2;
+    }
+}
+
+template <int BANK, typename T, bool NT>
+__global__ void __launch_bounds__(256) k_mas_lanes(DevData d, int force)
+{
+    constexpr int DIM = 3 * BANK, W = lane_tile_words(BANK, sizeof(T) == 4);
+    __shared__ float sR[4][DIM], sY[4][DIM];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int b = d.n_banks - 1 - ((int)blockIdx.x * 4 + wave);
+    if(b < 0) return;
+    const int kind = d.bank_kind[b], vec = d.bank_vec[b];
+    if(!(force || d.state[d.single ? 0 : d.bank_sys[b]].status == kRunning)) return;
+    uint32_t raw[W];
+    load_lane_tiles<BANK, T, NT>(d.minv, b, lane, raw);
+    float* R = sR[wave];
+    lane_bank_residual<BANK>(d, b, kind, vec, lane, R);
+    wave_sync();
+    float y[3];
+    int   at[3];
+    bool  mine;
+    lane_tile_product<BANK, T>(raw, R, sY[wave], lane, y, at, mine);
+    if(!mine) return;
+    const float sc = sizeof(T) == 4 ? 1.f : d.minv_scale[b];
+    float* dst = (kind == 0 ? d.z : d.Zc) + 3 * (long long)vec;
+#pragma unroll
+    for(int k = 0; k < 3; ++k) dst[at[k]] = y[k] * sc;
 }
 
 // ---- MAS local solve on MFMA (32-slot banks, FP16 / BF16 inverse) ---------
@@ -2779,9 +3024,12 @@ hipError_t launch_gal_gather(const double* fine, double* E, const int* ptr, cons
 
 size_t mas_bank_bytes(int bank, int precision)
 {
-    if(bank == 32 && precision != kPrecFp32) return (size_t)kTileBankHalves * 2;  // either layout fits
-    const size_t nblk = (size_t)bank * (bank + 1) / 2;
-    return nblk * (precision == kPrecFp32 ? 9 : 5) * 4;
+    // the largest of the layouts
+    const bool   f32   = precision == kPrecFp32;
+    const size_t nblk  = (size_t)bank * (bank + 1) / 2;
+    const size_t lanes = (size_t)lane_tile_values(bank, f32) * (f32 ? 4 : 2);
+    const size_t mfma  = bank == 32 && !f32 ? (size_t)kTileBankHalves * 2 : 0;
+    return std::max({nblk * (f32 ? 9 : 5) * 4, lanes, mfma});
 }
 
 hipError_t launch_mas_factor(const DevData& d, const double* E, const int* ent_ptr, const int* ent_pos,
@@ -2821,22 +3069,25 @@ hipError_t launch_mas_factor(const DevData& d, const double* E, const int* ent_p
     return hipSuccess;
 }
 
-int inverse_map_entries(int bank, int precision, bool tiles)
+int inverse_map_entries(int bank, int precision, int mas_waves)
 {
     const int nblk = bank * (bank + 1) / 2;
+    if(mas_waves == 2) return lane_tile_values(bank, precision == kPrecFp32);
     if(precision == kPrecFp32) return nblk * 9;
-    if(tiles && bank == 32) return kTileBankHalves;
+    if(mas_waves == 1 && bank == 32) return kTileBankHalves;
     return nblk * 10;
 }
 
-hipError_t launch_inverse_map(int bank, int precision, bool tiles, unsigned short* map, hipStream_t st)
+hipError_t launch_inverse_map(int bank, int precision, int mas_waves, unsigned short* map, hipStream_t st)
 {
-    const int n = inverse_map_entries(bank, precision, tiles);
+    const int n = inverse_map_entries(bank, precision, mas_waves);
+    const int layout = mas_waves == 2 ? kLaneTiles
+                       : mas_waves == 1 && bank == 32 && precision != kPrecFp32 ? kMfmaTiles : kByDiagonals;
     hipError_t e = hipMemsetAsync(map, 0xff, sizeof(unsigned short) * (size_t)n, st);
     if(e != hipSuccess) return e;
     const int ne = 3 * bank * (3 * bank + 1) / 2;
     const dim3 g((ne + 255) / 256);
-#define MASX_MAP(BK, T) hipLaunchKernelGGL((k_inverse_map<BK, T>), g, dim3(256), 0, st, map, tiles ? 1 : 0)
+#define MASX_MAP(BK, T) hipLaunchKernelGGL((k_inverse_map<BK, T>), g, dim3(256), 0, st, map, layout)
     if(bank == 32)
     {
         if(precision == kPrecFp16) MASX_MAP(32, __half);
@@ -2932,6 +3183,32 @@ hipError_t launch_mas_local(const DevData& d, int precision, int force, hipStrea
     if(d.n_banks <= 0) return hipSuccess;
     const bool mfma = d.bank == 32 && precision != kPrecFp32 && d.mas_waves == 1;
     const bool staged = precision == kPrecFp32 && (d.mas_waves == 5 || d.mas_waves == 9);
+    if(d.mas_waves == 2)
+    {
+        if(d.bank != 32 && d.bank != 16) return hipErrorInvalidValue;
+        const dim3 gl(blocks_for(d.n_banks, 4)), bl(256);
+#define MASX_LANES(BK, T)                                                              \
+    do                                                                                 \
+    {                                                                                  \
+        if(d.mas_nt) MASX_DISPATCH((k_mas_lanes<BK, T, true>), gl, bl, d, force);      \
+        else MASX_DISPATCH((k_mas_lanes<BK, T, false>), gl, bl, d, force);             \
+    } while(0)
+        if(d.bank == 32)
+        {
+            if(precision == kPrecFp16) MASX_LANES(32, __half);
+            else if(precision == kPrecBf16) MASX_LANES(32, __hip_bfloat16);
+            else MASX_LANES(32, float);
+        }
+        else
+        {
+            if(precision == kPrecFp16) MASX_LANES(16, __half);
+            else if(precision == kPrecBf16) MASX_LANES(16, __hip_bfloat16);
+            else MASX_LANES(16, float);
+        }
+#undef MASX_LANES
+        MASX_CHECK_LAUNCH();
+        return hipSuccess;
+    }
     if(!mfma && !staged && d.mas_waves != 4 && d.mas_waves != 8) return hipErrorInvalidValue;
     const int bpw = 64 / d.bank;
     const dim3 g(blocks_for(d.n_banks, bpw)), b(256);

@@ -1,5 +1,6 @@
 // Host orchestrator of the MAS-PCG solve (see solver.hpp).
 #include "solver.hpp"
+#include "lane_tiles.hpp"
 #include "mas_tiles.hpp"
 #include "phase_timer.hpp"
 
@@ -240,25 +241,23 @@ void Solver::set_spmv_tiling(int entries_per_thread)
     }
 }
 
-// From this many banks on the MAS local kernel defaults to the MFMA kernel
-// (half-precision 32-slot banks) or the LDS-staged FP32 kernel; below, the
-// register-fed VALU kernel's shorter latency wins (measured on 2,270 and
-// 91,066 banks).
-constexpr int kMfmaAutoBanks = 16384;
+// From this many banks the inverses outgrow the caches by far: streamed.
+constexpr int kStreamedBanks = 16384;
 
-int Solver::effective_mas_waves() const
+// The variant that a setting selects among the block-diagonal and MFMA
+// kernels (the ones a caller can ask for); automatic is the lane-tile kernel,
+// and stands here for MFMA on large half-precision batches, else 4 waves.
+int Solver::settable_variant(int waves) const
 {
     const bool mfma_ok = plan_.bank == 32 && precision_ != kPrecFp32;
     const bool fp32    = precision_ == kPrecFp32;
-    if(mas_waves_ == 1) return mfma_ok ? 1 : 4;
-    if(mas_waves_ == 4 || mas_waves_ == 8) return mas_waves_;
-    if(mas_waves_ == 5 || mas_waves_ == 9) return fp32 ? mas_waves_ : mas_waves_ - 1;  // LDS staging is FP32's
-    // automatic: on large batches the MFMA kernel (half) or the LDS-staged
-    // FP32 kernel stream the inverse fastest; on a few thousand banks the
-    // register-fed 4-wave kernel's shorter latency wins
-    if(plan_.n_banks >= kMfmaAutoBanks) return mfma_ok ? 1 : (fp32 ? 9 : 4);
-    return 4;
+    if(waves == 1) return mfma_ok ? 1 : 4;
+    if(waves == 4 || waves == 8) return waves;
+    if(waves == 5 || waves == 9) return fp32 ? waves : waves - 1;  // LDS staging is FP32's
+    return plan_.n_banks >= kStreamedBanks && mfma_ok ? 1 : 4;
 }
+
+int Solver::effective_mas_waves() const { return mas_waves_ == 0 ? 2 : settable_variant(mas_waves_); }
 
 void Solver::set_mas_waves(int waves)
 {
@@ -266,21 +265,30 @@ void Solver::set_mas_waves(int waves)
         throw std::invalid_argument(
             "MAS local variant must be 0 (automatic), 1 (MFMA), 4 or 8 (waves per workgroup), 5 or 9 (4 or 8 waves, "
             "FP32 inverse staged through LDS)");
-    const bool tiles_before = effective_mas_waves() == 1;
+    const bool mfma_before = settable_variant(mas_waves_) == 1;
+    const int  before      = effective_mas_waves();
     mas_waves_    = waves;
     dd_.mas_waves = effective_mas_waves();
-    if(built_ && (dd_.mas_waves == 1) != tiles_before) built_ = false;  // the inverse is in the other layout
     if(graph_exec_) (void)hipGraphExecDestroy(graph_exec_);
     graph_exec_ = nullptr;
+    if(!built_) return;
+    if((settable_variant(waves) == 1) != mfma_before)
+        built_ = false;  // the inverse is in the other layout: the caller builds again
+    else if((before == 2) != (dd_.mas_waves == 2) || (before == 1) != (dd_.mas_waves == 1))
+        build(precision_, nullptr);  // to or from lane tiles
 }
 
 Solver::Tiling Solver::autotune_mas(int reps)
 {
     if(!built_) throw std::runtime_error("build() must precede autotune");
-    if(plan_.n_banks == 0) return Tiling{effective_mas_waves(), 0.0};
-    // the automatic choice first; another variant replaces the best only when
-    // it is more than 2 % faster, so near-ties keep one choice from run to run
-    const int first = effective_mas_waves();
+    if(plan_.n_banks == 0) return Tiling{settable_variant(mas_waves_), 0.0};
+    // the automatic kernel stays unless a variant that can be set is more than
+    // 2 % faster; among those one replaces the best by the same rule, so
+    // near-ties keep one choice from run to run
+    set_mas_waves(0);
+    if(!built_) build(precision_, nullptr);
+    const double automatic = time_kernel(0, reps);
+    const int first = settable_variant(0);
     std::vector<int> cand = {first};
     for(const int w : {1, 4, 8, 5, 9})
     {
@@ -297,7 +305,7 @@ Solver::Tiling Solver::autotune_mas(int reps)
         const double ms = time_kernel(0, reps);
         if(ms < 0.98 * best.ms) best = Tiling{w, ms};
     }
-    set_mas_waves(best.entries);
+    set_mas_waves(best.ms < 0.98 * automatic ? best.entries : 0);
     if(!built_) build(precision_, nullptr);
     return best;
 }
@@ -403,6 +411,19 @@ void Solver::setup()
     d_bank_vec_.upload(P.bank_vec, st);
     d_bank_sys_.upload(P.bank_sys, st);
     d_bank_kind_.upload(P.bank_kind, st);
+    {
+        // nodes that exist in each coarse bank: every one is a level-1 node or
+        // the ancestor of one
+        std::vector<int> live(P.n_banks - P.n_fine_banks, 0);
+        const int n_comp = P.n_banks > 0 ? P.comp_ptr[P.n_fine_banks] : 0;
+        for(int c = 0; c < n_comp; ++c)
+            for(int k = 0; k < 8; ++k)
+            {
+                const int a = P.anc[8 * (size_t)P.comp_parent[c] + k];
+                if(a >= 0) live[a / P.bank] = std::max(live[a / P.bank], a % P.bank + 1);
+            }
+        d_bank_live_.upload(live, st);
+    }
     d_comp_ptr_.upload(P.comp_ptr, st);
     d_comp_mask_.upload(P.comp_mask, st);
     d_comp_parent_.upload(P.comp_parent, st);
@@ -603,6 +624,7 @@ void Solver::make_devdata()
     d.bank = P.bank;
     d.n_banks = P.n_banks;
     d.mas_waves = effective_mas_waves();
+    d.mas_nt = P.n_banks >= kStreamedBanks ? 1 : 0;
     d.n_fine_banks = P.n_fine_banks;
     d.nnz = P.nnz;
     d.nnz_s = spmv_layout_.total;
@@ -640,6 +662,7 @@ void Solver::make_devdata()
     d.bank_vec = d_bank_vec_.ptr;
     d.bank_sys = d_bank_sys_.ptr;
     d.bank_kind = d_bank_kind_.ptr;
+    d.bank_live = d_bank_live_.ptr;
     d.comp_ptr = d_comp_ptr_.ptr;
     d.comp_mask = d_comp_mask_.ptr;
     d.comp_parent = d_comp_parent_.ptr;
@@ -829,12 +852,11 @@ void Solver::build(int precision, hipStream_t user)
     const Plan& P = plan_;
     {
         // the factor writes the inverse through this layout's map
-        const bool tiles = P.bank == 32 && precision_ != kPrecFp32 && dd_.mas_waves == 1;
-        const int  key   = (P.bank * 4 + precision_) * 2 + (tiles ? 1 : 0);
+        const int key = (P.bank * 4 + precision_) * 16 + dd_.mas_waves;
         if(key != inv_map_key_ && P.n_banks > 0)
         {
-            d_inv_map_.alloc((size_t)inverse_map_entries(P.bank, precision_, tiles));
-            MASX_HIP(launch_inverse_map(P.bank, precision_, tiles, d_inv_map_.ptr, st));
+            d_inv_map_.alloc((size_t)inverse_map_entries(P.bank, precision_, dd_.mas_waves));
+            MASX_HIP(launch_inverse_map(P.bank, precision_, dd_.mas_waves, d_inv_map_.ptr, st));
             inv_map_key_ = key;
         }
         dd_.inv_map = d_inv_map_.ptr;
@@ -1062,8 +1084,11 @@ void Solver::download_inverse(std::vector<float>& out)
         MASX_HIP(hipMemcpy(scale.data(), d_minv_scale_.ptr, sizeof(float) * plan_.n_banks, hipMemcpyDeviceToHost));
     const size_t bank_bytes = mas_bank_bytes(B, precision_);
     // words per bank as the local kernels index them: FP32 9 per block, the
-    // half block-diagonal layout 5 per block, the MFMA tiles kTileBankHalves / 2
-    const size_t stride_words = precision_ == kPrecFp32 ? nblk * 9
+    // half block-diagonal layout 5 per block, the MFMA tiles kTileBankHalves / 2,
+    // the lane tiles 64 lanes' words
+    const bool f32 = precision_ == kPrecFp32, lanes = dd_.mas_waves == 2;
+    const size_t stride_words = lanes ? (size_t)64 * lane_tile_words(B, f32)
+                                : precision_ == kPrecFp32 ? nblk * 9
                                 : (B == 32 && dd_.mas_waves == 1) ? (size_t)kTileBankHalves / 2
                                                                    : nblk * 5;
     std::vector<uint32_t> raw((size_t)plan_.n_banks * bank_bytes / 4);
@@ -1096,7 +1121,16 @@ void Solver::download_inverse(std::vector<float>& out)
                 for(int c = 0; c < 9; ++c)
                 {
                     float v;
-                    if(precision_ == kPrecFp32)
+                    if(lanes)
+                    {
+                        const int r = 3 * I + c / 3, col = 3 * (I + dd) + c % 3;
+                        const int p = lane_tile_slot(B, f32, std::max(r, col), std::min(r, col));
+                        if(f32)
+                            std::memcpy(&v, &bw[p], 4);
+                        else
+                            v = half_to_float(p % 2 ? (bw[p / 2] >> 16) : (bw[p / 2] & 0xffffu)) * scale[b];
+                    }
+                    else if(precision_ == kPrecFp32)
                     {
                         std::memcpy(&v, &bw[9 * off + c * len + I], 4);
                     }

@@ -116,18 +116,18 @@ class Solver
     // banks on); takes effect at the next build()
     void set_factor_waves(int waves);
     int  factor_waves() const { return effective_factor_waves(); }
-    // MAS local kernel: 4 or 8 waves per workgroup (VALU; each workgroup holds
-    // 64 / bank banks, its waves split their block diagonals), 5 or 9 (the
-    // same with 4 or 8 waves, the FP32 inverse staged through LDS with
-    // 16-byte loads; half precision falls back to 4 or 8), 1 (the MFMA
-    // kernel, one wave per bank: FP16 / BF16 inverses of 32-slot banks; other
-    // cases fall back to 4), or 0 (automatic: from kMfmaAutoBanks banks on
-    // MFMA for half-precision 32-slot banks and 9 for FP32, else 4).  A change that moves the
-    // half-precision inverse between the two layouts needs a new build().
+    // MAS local kernel: 0 (automatic: lane tiles, one wave per bank), 4 or 8
+    // waves per workgroup (block diagonals; each workgroup holds 64 / bank
+    // banks, its waves split their block diagonals), 5 or 9 (the same with 4
+    // or 8 waves, the FP32 inverse staged through LDS with 16-byte loads;
+    // half precision falls back to 4 or 8), 1 (the MFMA kernel, one wave per
+    // bank: FP16 / BF16 inverses of 32-slot banks; other cases fall back to
+    // 4).  After a build, a change between the MFMA and the block-diagonal
+    // layout leaves the solver unbuilt; one to or from lane tiles builds again.
     void set_mas_waves(int waves);
-    int  mas_waves() const { return effective_mas_waves(); }
-    // times every MAS local variant the built precision has and keeps the
-    // fastest (rebuilding when the variant's inverse layout differs)
+    int  mas_waves() const { return settable_variant(mas_waves_); }
+    // times the settable MAS local variants of the built precision, returns the
+    // fastest and sets it if it beats the automatic kernel
     Tiling autotune_mas(int reps);
     // average device time of one kernel of the iteration over `reps` launches
     // (0 MAS local, 1 preconditioner finish, 2 SpMV, 3 update), milliseconds
@@ -162,6 +162,7 @@ class Solver
     int  entries_    = 4;
     int  mas_waves_  = 0;
     int  effective_mas_waves() const;
+    int  settable_variant(int waves) const;
     int  spmv_loads_ = 0;
     bool effective_spmv_nt() const;
     int  factor_waves_ = 0;
@@ -183,7 +184,7 @@ class Solver
     DeviceArray<float>     d_x_, d_r_, d_z_, d_p0_, d_p1_, d_Ap_, d_rt_, d_Rc_, d_Zc_, d_part_deep_;
     DeviceArray<char>      d_minv_;
     DeviceArray<float>     d_minv_scale_;
-    DeviceArray<int>       d_bank_vec_, d_bank_sys_, d_bank_kind_, d_comp_ptr_, d_comp_parent_;
+    DeviceArray<int>       d_bank_vec_, d_bank_sys_, d_bank_kind_, d_bank_live_, d_comp_ptr_, d_comp_parent_;
     DeviceArray<uint32_t>  d_comp_mask_;
     DeviceArray<int>       d_deep_ptr_, d_deep_list_, d_row_l1_, d_anc_, d_bank_ugroup_, d_ugroup_, d_comp_dslot_;
     DeviceArray<int>       d_gal_ptr_, d_gal_src_, d_ent_ptr_, d_ent_pos_, d_ent_src_;

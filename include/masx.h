@@ -196,15 +196,18 @@ int masx_autotune(masx_solver* s, int reps, int* entries_per_thread, double* ms)
 int masx_set_spmv_loads(masx_solver* s, int mode);
 /* *nontemporal: whether the SpMV currently uses nontemporal loads. */
 int masx_spmv_loads_used(masx_solver* s, int* nontemporal);
-/* MAS local solve variant.  waves = 4 or 8: the VALU kernel, that many
+/* MAS local solve variant.  0 (the default): one wave per bank on lane tiles
+ * (every element of the inverse in one lane's registers).  The others:
+ * waves = 4 or 8: the block-diagonal VALU kernel, that many
  * waves per workgroup sharing the block diagonals of its banks; 5 or 9: the
  * same with 4 or 8 waves, the workgroup's FP32 inverses staged through LDS
  * with 16-byte loads (half precision runs 4 or 8); 1: the MFMA kernel, one
- * wave per bank (FP16 / BF16 inverses of 32-slot banks; other cases run 4);
- * 0 (the default): from 16,384 banks on MFMA for half-precision 32-slot
- * banks and 9 for FP32, else 4.  The two kernels store a half-precision inverse in
- * different layouts: a change between them needs a new masx_build before the
- * next solve (masx_solve reports the missing build). */
+ * wave per bank (FP16 / BF16 inverses of 32-slot banks; other cases run 4).
+ * Each kind stores the inverse in a layout of its own.  A change between
+ * variants after a build builds again by itself, except between 1 and 4, 5,
+ * 8 or 9 on a half-precision inverse (0 counts as 1 from 16,384 such
+ * 32-slot banks on, else as 4): that needs a new masx_build before the next
+ * solve (masx_solve reports the missing build). */
 int masx_set_mas_waves(masx_solver* s, int waves);
 /* MAS factor (the dense assembly and FP64 inverse of every bank at
  * masx_build): waves = 1, one wave per bank (more banks per SIMD; the faster
@@ -214,10 +217,11 @@ int masx_set_mas_waves(masx_solver* s, int waves);
  * counterpart in the reference (__inverse6_P96x96,
  * TraditionalMAS32Preconditioner.cu:1099-1147, has one form). */
 int masx_set_factor_waves(masx_solver* s, int waves);
-/* Times every MAS local variant of the built precision (`reps` launches
- * each; for half-precision 32-slot banks 1, 4 and 8, else 4 and 8), keeps the
- * fastest (rebuilding the preconditioner for a layout change) and reports it
- * and its time per launch (ms).  Leaves the iteration state frozen like
+/* Times the MAS local variants of the built precision (`reps` launches
+ * each; for half-precision 32-slot banks 1, 4 and 8, else 4, 8, 5 and 9),
+ * reports the fastest of them and its time per launch (ms), and sets it if it
+ * beats the automatic kernel (0), which stays otherwise; the preconditioner is
+ * built again for a layout change.  Leaves the iteration state frozen like
  * masx_autotune. */
 int masx_autotune_mas(masx_solver* s, int reps, int* waves, double* ms);
 /* Average execution time of one kernel (0 MAS local, 1 preconditioner finish,
