@@ -100,12 +100,12 @@ struct DevData
     const int*      comp_ptr;
     const uint32_t* comp_mask;
     const int*      comp_parent;
-    const int*      deep_ptr;    // level >= 2 coarse node -> its update-group partial slots
-    const int*      deep_list;
+    const int*      deep_ptr;    // level >= 2 coarse node -> its update-group partials in part_deep
+    const int*      deep_pos;    // update-group slot -> its place in part_deep
     const int*      bank_ugroup; // fine bank -> update group
     const int4*     ugroup;      // {slot base, slot count, component begin, component end}
     const int*      comp_dslot;  // 4 per fine-bank component: group-local slot per deep level, -1 none
-    float*          part_deep;   // float3 per slot, written by the update kernel
+    float*          part_deep;   // float3 per slot, node by node, written by the update kernel
     const int*      row_l1;      // per internal row: its level-1 node, -1 none
     const int*      anc;         // 8 per coarse node (used for level-1 nodes): itself and its ancestors, -1 padded
     // ABD and diagonal block-Jacobi

@@ -258,6 +258,7 @@ __device__ double sys_sum(const double* part, int2 r, double* smem)
 __device__ __forceinline__ double partial_share(const double* part, int2 r)
 {
     const int b = r.x, e = r.y;
+    if(e - b <= 256) return b + (int)threadIdx.x < e ? part[b + (int)threadIdx.x] : 0.0;  // one each: no loop to issue
     double v = 0.0;
 #pragma unroll 1
     for(int i = b + (int)threadIdx.x; i < e; i += 8 * 256)
@@ -1323,7 +1324,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4,
     if(tid < 3) sR[64 * 3 + tid] = 0.f;
     // level >= 2: R(node) = sum of the partials the update kernel formed for
     // it, one per 256-row group holding some of its level-1 descendants.  The
-    // lists of a bank's consecutive nodes are contiguous in deep_list; they
+    // partials of a bank's consecutive nodes are contiguous; they
     // pass through LDS in chunks with every load of a chunk in flight, then
     // each node's TPN threads sum its entries in list order.
 #pragma unroll 1
@@ -1345,7 +1346,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4,
             for(int j = 0; j < CHUNK / THREADS; ++j)
             {
                 const int e = tid + THREADS * j;
-                src[j] = e < n ? d.deep_list[base + e] : -1;
+                src[j] = e < n ? base + e : -1;
             }
 #pragma unroll
             for(int j = 0; j < CHUNK / THREADS; ++j)
@@ -1514,7 +1515,8 @@ __device__ __forceinline__ V ld_inverse(const V* p)
 
 // A lane's values of its bank as stored: 16-byte groups of every lane, then
 // the rest of a few values per lane.
-template <int BANK, typename T, bool NT>
+// BEGIN, END: the groups to load (the rest counts as the last).
+template <int BANK, typename T, bool NT, int BEGIN, int END>
 __device__ __forceinline__ void load_lane_tiles(const void* minv, int bank, int lane,
                                                 uint32_t (&raw)[lane_tile_words(BANK, sizeof(T) == 4)])
 {
@@ -1522,11 +1524,12 @@ __device__ __forceinline__ void load_lane_tiles(const void* minv, int bank, int 
     constexpr int W = lane_tile_words(BANK, F32), Q = W / 4, REM = W % 4;
     const char* base = reinterpret_cast<const char*>(minv) + (size_t)bank * (lane_tile_values(BANK, F32) * sizeof(T));
 #pragma unroll
-    for(int q = 0; q < Q; ++q)
+    for(int q = BEGIN; q < (END < Q ? END : Q); ++q)
     {
         const uint4 v = ld_inverse<NT>(reinterpret_cast<const uint4*>(base) + 64 * q + lane);
         raw[4 * q] = v.x; raw[4 * q + 1] = v.y; raw[4 * q + 2] = v.z; raw[4 * q + 3] = v.w;
     }
+    if(END <= Q) return;
     const uint32_t* rest = reinterpret_cast<const uint32_t*>(base) + 256 * Q + REM * lane;
 #pragma unroll
     for(int q = 0; q < REM; ++q) raw[4 * Q + q] = ld_inverse<NT>(rest + q);
@@ -1543,7 +1546,8 @@ __device__ __forceinline__ float lane_tile_value(const uint32_t (&raw)[W], int s
 
 // z = (stored inverse) R over the bank's dim values; R and Y: dim floats of the
 // wave's LDS each.  Afterwards lanes with `mine` hold z[at[k]] in y[k].
-template <int BANK, typename T, int W>
+// Only the tiles of the first 8 A rows are used (the rest of R is zero).
+template <int BANK, typename T, int A, int W>
 __device__ __forceinline__ void lane_tile_product(const uint32_t (&raw)[W], const float* R, float* Y, int lane,
                                                   float (&y)[3], int (&at)[3], bool& mine)
 {
@@ -1554,12 +1558,12 @@ __device__ __forceinline__ void lane_tile_product(const uint32_t (&raw)[W], cons
 #pragma unroll
     for(int a = 0; a < TT; ++a)
     {
-        rr[a] = R[ty + 8 * a];
-        rc[a] = R[tx + 8 * a];
+        rr[a] = a < A ? R[ty + 8 * a] : 0.f;
+        rc[a] = a < A ? R[tx + 8 * a] : 0.f;
         yr[a] = yc[a] = 0.f;
     }
 #pragma unroll
-    for(int a = 0; a < TT; ++a)
+    for(int a = 0; a < A; ++a)
 #pragma unroll
         for(int b = 0; b <= a; ++b)
         {
@@ -1631,9 +1635,9 @@ __device__ __forceinline__ void lane_tile_product(const uint32_t (&raw)[W], cons
     }
 }
 
-// Residual of one bank (dim values) into the wave's LDS.
+// Residual of one bank (dim values) of m nodes into the wave's LDS.
 template <int BANK>
-__device__ __forceinline__ void lane_bank_residual(const DevData& d, int bank, int kind, int vec, int lane, float* R)
+__device__ __forceinline__ void lane_bank_residual(const DevData& d, int kind, int vec, int m, int lane, float* R)
 {
     if(kind < 2)
     {
@@ -1643,7 +1647,6 @@ __device__ __forceinline__ void lane_bank_residual(const DevData& d, int bank, i
             if(i + lane < 3 * BANK) R[i + lane] = r[i + lane];
         return;
     }
-    const int m = d.bank_live[bank - d.n_fine_banks];
     int P = 64;  // lanes per live node: a power of two
     while(P * m > 64) P >>= 1;
     const int node = lane / P, sub = lane % P;
@@ -1654,8 +1657,8 @@ __device__ __forceinline__ void lane_bank_residual(const DevData& d, int bank, i
 #pragma unroll 4
         for(int k = d.deep_ptr[vec + node] + sub; k < end; k += P)
         {
-            const long long c = 3 * (long long)d.deep_list[k];
-            a0 += d.part_deep[c]; a1 += d.part_deep[c + 1]; a2 += d.part_deep[c + 2];
+            const float* c = d.part_deep + 3 * (long long)k;
+            a0 += c[0]; a1 += c[1]; a2 += c[2];
         }
     }
     for(int off = P >> 1; off > 0; off >>= 1)
@@ -1671,6 +1674,12 @@ __device__ __forceinline__ void lane_bank_residual(const DevData& d, int bank, i
     }
 }
 
+// A coarse bank of few nodes (the upper levels' are mostly empty): only its
+// first kFewTiles tile rows are loaded and used.
+constexpr int kFewTiles = 4;
+template <typename T>
+constexpr int kFewGroups = (kFewTiles * (kFewTiles + 1) / 2 * (int)sizeof(T) + 15) / 16;
+
 template <int BANK, typename T, bool NT>
 __global__ void __launch_bounds__(256) k_mas_lanes(DevData d, int force)
 {
@@ -1681,15 +1690,21 @@ __global__ void __launch_bounds__(256) k_mas_lanes(DevData d, int force)
     if(b < 0) return;
     const int kind = d.bank_kind[b], vec = d.bank_vec[b];
     if(!(force || d.state[d.single ? 0 : d.bank_sys[b]].status == kRunning)) return;
+    const int  live = kind == 0 ? BANK : d.bank_live[b - d.n_fine_banks];
+    const bool few  = 3 * live <= 8 * kFewTiles;
     uint32_t raw[W];
-    load_lane_tiles<BANK, T, NT>(d.minv, b, lane, raw);
+    load_lane_tiles<BANK, T, NT, 0, kFewGroups<T>>(d.minv, b, lane, raw);
+    if(!few) load_lane_tiles<BANK, T, NT, kFewGroups<T>, W>(d.minv, b, lane, raw);
     float* R = sR[wave];
-    lane_bank_residual<BANK>(d, b, kind, vec, lane, R);
+    lane_bank_residual<BANK>(d, kind, vec, live, lane, R);
     wave_sync();
     float y[3];
     int   at[3];
     bool  mine;
-    lane_tile_product<BANK, T>(raw, R, sY[wave], lane, y, at, mine);
+    if(few)
+        lane_tile_product<BANK, T, kFewTiles>(raw, R, sY[wave], lane, y, at, mine);
+    else
+        lane_tile_product<BANK, T, LaneGrid<BANK>::T>(raw, R, sY[wave], lane, y, at, mine);
     if(!mine) return;
     const float sc = sizeof(T) == 4 ? 1.f : d.minv_scale[b];
     float* dst = (kind == 0 ? d.z : d.Zc) + 3 * (long long)vec;
@@ -1855,7 +1870,7 @@ __global__ void __launch_bounds__(256) k_mas_local_mfma(DevData d, int force)
             for(int j = 0; j < CHUNK / 256; ++j)
             {
                 const int e = tid + 256 * j;
-                src[j] = e < n ? d.deep_list[base + e] : -1;
+                src[j] = e < n ? base + e : -1;
             }
 #pragma unroll
             for(int j = 0; j < CHUNK / 256; ++j)
@@ -2637,6 +2652,7 @@ __global__ void __launch_bounds__(256) k_update(DevData d, const float* __restri
     // lane j of a bank holds the bank's component cb + j (at most one per lane)
     const int blane = threadIdx.x & (d.bank - 1);
     const bool has_comp = restrict_rows && cb + blane < ce;
+    const int deep_pos = (int)threadIdx.x < grp.y ? d.deep_pos[grp.x + (int)threadIdx.x] : 0;
     uint32_t my_mask = 0;
     int      my_parent = 0;
     int4     my_ds = make_int4(-1, -1, -1, -1);
@@ -2753,7 +2769,7 @@ __global__ void __launch_bounds__(256) k_update(DevData d, const float* __restri
                         ax += v[k][0]; ay += v[k][1]; az += v[k][2];
                     }
             }
-            const long long o = 3 * (long long)(grp.x + t);
+            const long long o = 3 * (long long)(t == (int)threadIdx.x ? deep_pos : d.deep_pos[grp.x + t]);
             d.part_deep[o] = ax; d.part_deep[o + 1] = ay; d.part_deep[o + 2] = az;
         }
     }

@@ -428,7 +428,12 @@ void Solver::setup()
     d_comp_mask_.upload(P.comp_mask, st);
     d_comp_parent_.upload(P.comp_parent, st);
     d_deep_ptr_.upload(P.deep_ptr, st);
-    d_deep_list_.upload(P.deep_list, st);
+    {
+        // the update kernel stores each partial at its place in the node lists
+        std::vector<int> pos(P.deep_list.size());
+        for(size_t e = 0; e < pos.size(); ++e) pos[P.deep_list[e]] = (int)e;
+        d_deep_pos_.upload(pos, st);
+    }
     d_bank_ugroup_.upload(P.bank_ugroup, st);
     d_ugroup_.upload(P.ugroup, st);
     d_comp_dslot_.upload(P.comp_dslot, st);
@@ -667,7 +672,7 @@ void Solver::make_devdata()
     d.comp_mask = d_comp_mask_.ptr;
     d.comp_parent = d_comp_parent_.ptr;
     d.deep_ptr = d_deep_ptr_.ptr;
-    d.deep_list = d_deep_list_.ptr;
+    d.deep_pos = d_deep_pos_.ptr;
     d.bank_ugroup = d_bank_ugroup_.ptr;
     d.ugroup = reinterpret_cast<const int4*>(d_ugroup_.ptr);
     d.comp_dslot = d_comp_dslot_.ptr;
