@@ -333,41 +333,115 @@ __global__ void __launch_bounds__(256) k_pack_abd(DevData d, const int* __restri
         for(int j = 0; j < 3; ++j) out[12 * i + j] = (float)acc[3 * i + j];
 }
 
-// Upper FP64 blocks (col-major) -> FP32 SoA planes of the SpMV layout, one
-// thread per entry so the plane writes are contiguous; an entry marked
-// transposed takes its upper block's transpose, a padding entry zeros.
+// Upper FP64 blocks (col-major) -> FP32 SoA planes of the SpMV layout; an
+// entry marked transposed takes its upper block's transpose, a padding entry
+// zeros.  Nine lanes read an entry's 72 contiguous bytes, the values turn over
+// in LDS and leave plane by plane in whole lines (8 M entries of 685,427
+// vertices: 169 us with a thread per entry, 154 this way).
+constexpr int kPackEntries = 28 * 9;
 __global__ void __launch_bounds__(256) k_pack_values(DevData d)
 {
-    const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if(e >= d.nnz_s) return;
-    const int code = d.sy_src[e];
+    constexpr int K = kPackEntries / 28;
+    __shared__ float sV[kPackEntries * 9];
+    const int tid = threadIdx.x, g = tid / 9, q = tid % 9, qt = q / 3 + 3 * (q % 3);
+    const long long e0 = (long long)blockIdx.x * kPackEntries;
+    const int n = (int)min((long long)kPackEntries, d.nnz_s - e0);
+    if(tid < 252)
+    {
+        int    code[K];
+        double v[K];
+#pragma unroll
+        for(int k = 0; k < K; ++k) code[k] = d.sy_src[e0 + min(g + 28 * k, n - 1)];
+#pragma unroll
+        for(int k = 0; k < K; ++k)
+        {
+            // row-major value q of the block as is (column-major) or transposed
+            const bool pad = code[k] == kSpmvPadSrc;
+            const long long src = pad ? 0 : code[k] & 0x7fffffff;
+            v[k] = pad ? 0.0 : d.vals64[9 * src + (code[k] >= 0 ? qt : q)];
+        }
+#pragma unroll
+        for(int k = 0; k < K; ++k) sV[9 * (g + 28 * k) + q] = (float)v[k];
+    }
+    __syncthreads();
     float* planes = const_cast<float*>(d.vals32);
-    if(code == kSpmvPadSrc)
-    {
+    if(tid < n)
 #pragma unroll
-        for(int q = 0; q < 9; ++q) planes[q * d.plane + e] = 0.f;
-        return;
-    }
-    const double* B = d.vals64 + 9 * (long long)(code & 0x7fffffff);
-    if(code >= 0)
-    {
-#pragma unroll
-        for(int i = 0; i < 3; ++i)
-#pragma unroll
-            for(int j = 0; j < 3; ++j) planes[(3 * i + j) * d.plane + e] = (float)B[i + 3 * j];
-    }
-    else
-    {
-#pragma unroll
-        for(int i = 0; i < 3; ++i)
-#pragma unroll
-            for(int j = 0; j < 3; ++j) planes[(3 * i + j) * d.plane + e] = (float)B[j + 3 * i];
-    }
+        for(int c = 0; c < 9; ++c) planes[c * d.plane + e0 + tid] = sV[9 * tid + c];
 }
 
-// Galerkin coarse entries of one level: E[e] = sum of its mapped sources
-// (as is, transposed, or B + B^T).  G lanes per entry stride over its source
-// list; their sums meet in a fixed shuffle tree.
+// Galerkin coarse entries of one level: E[e] = sum of its mapped sources (as
+// is, transposed, or B + B^T).  As in the Hessian's gather, a workgroup owns 32
+// consecutive entries and walks their sources (consecutive in the list) in
+// chunks: nine lanes read a source's 72 contiguous bytes into LDS, in the order
+// of its mode, and the 288 entry values are summed from there in source
+// order, so the work is even whatever an entry's count (about 8 off the
+// diagonal, 120 on it).  For the large levels with short lists: the first of
+// 685,427 vertices takes 138 us this way, 2.9 TB/s, while a level of a few
+// thousand entries leaves the chip empty (40^3: 17 us for the three levels'
+// mean against 12 us with lanes per entry, k_gal_gather).
+constexpr int kGalEntries = 32, kGalChunk = 28 * 9;
+constexpr int kGalLinesMin = 65536;  // entries: eight workgroups per CU
+__global__ void __launch_bounds__(256) k_gal_gather_lines(const double* __restrict__ fine, double* E,
+                                                          const int* __restrict__ ptr, const int* __restrict__ src,
+                                                          int e0, int e1, int src_is_fine)
+{
+    constexpr int K = kGalChunk / 28, OWN = (9 * kGalEntries + 255) / 256;
+    __shared__ double sE[9 * kGalChunk];
+    const int tid = threadIdx.x, b0 = e0 + xcd_tile(blockIdx.x, gridDim.x) * kGalEntries;
+    const int ne = min(kGalEntries, e1 - b0);
+    const int k0 = ptr[b0], total = ptr[b0 + ne] - k0;
+    double acc[OWN];
+    int    lo[OWN], hi[OWN];
+#pragma unroll
+    for(int m = 0; m < OWN; ++m)
+    {
+        const int o = tid + 256 * m;
+        acc[m] = 0.0;
+        lo[m] = o < 9 * ne ? ptr[b0 + o / 9] - k0 : 0;
+        hi[m] = o < 9 * ne ? ptr[b0 + o / 9 + 1] - k0 : 0;
+    }
+    const int g = tid / 9, q = tid % 9, qt = q / 3 + 3 * (q % 3);
+    // value q of the source (row-major): fine blocks are column-major, coarse ones row-major
+    const int as_is = src_is_fine ? qt : q, turned = src_is_fine ? q : qt;
+    const double* S = src_is_fine ? fine : E;
+#pragma unroll 1
+    for(int c0 = 0; c0 < total; c0 += kGalChunk)
+    {
+        const int n = min(kGalChunk, total - c0);
+        if(tid < 252)
+        {
+            int    code[K];
+            double v[K];
+#pragma unroll
+            for(int k = 0; k < K; ++k) code[k] = src[k0 + c0 + min(g + 28 * k, n - 1)];
+#pragma unroll
+            for(int k = 0; k < K; ++k)
+            {
+                const double* B = S + 9 * (long long)(code[k] >> 2);
+                v[k] = B[(code[k] & 3) == 1 ? turned : as_is];
+                if((code[k] & 3) == 2) v[k] += B[turned];
+            }
+#pragma unroll
+            for(int k = 0; k < K; ++k) sE[9 * (g + 28 * k) + q] = v[k];
+        }
+        __syncthreads();
+#pragma unroll
+        for(int m = 0; m < OWN; ++m)
+        {
+            const int b = max(lo[m], c0) - c0, e = min(hi[m], c0 + n) - c0, c = (tid + 256 * m) % 9;
+#pragma unroll 4
+            for(int k = b; k < e; ++k) acc[m] += sE[9 * k + c];
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for(int m = 0; m < OWN; ++m)
+        if(tid + 256 * m < 9 * ne) E[9 * (long long)b0 + tid + 256 * m] = acc[m];
+}
+
+// The same for few entries (G = 16) or long lists (G = 64): G lanes per entry
+// stride over its list; their sums meet in a fixed shuffle tree.
 template <int G>
 __global__ void __launch_bounds__(256) k_gal_gather(const double* fine, double* E, const int* ptr, const int* src,
                                                     int e0, int e1, int src_is_fine)
@@ -3007,7 +3081,7 @@ static inline unsigned blocks_for(long long n, int b) { return (unsigned)((n + b
 hipError_t launch_pack_values(const DevData& d, hipStream_t st)
 {
     if(d.nnz_s <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_pack_values, dim3(blocks_for(d.nnz_s, 256)), dim3(256), 0, st, d);
+    hipLaunchKernelGGL(k_pack_values, dim3(blocks_for(d.nnz_s, kPackEntries)), dim3(256), 0, st, d);
     MASX_CHECK_LAUNCH();
     return hipSuccess;
 }
@@ -3023,17 +3097,18 @@ hipError_t launch_pack_abd(const DevData& d, const int* cp_body, const int* cp_s
 }
 
 hipError_t launch_gal_gather(const double* fine, double* E, const int* ptr, const int* src, int e0, int e1,
-                             int src_is_fine, int lanes, hipStream_t st)
+                             int src_is_fine, bool long_lists, hipStream_t st)
 {
     if(e1 <= e0) return hipSuccess;
-    if(lanes == 64)
+    if(long_lists)
         hipLaunchKernelGGL(k_gal_gather<64>, dim3(blocks_for(e1 - e0, 4)), dim3(256), 0, st, fine, E, ptr, src, e0,
                            e1, src_is_fine);
-    else if(lanes == 16)
+    else if(e1 - e0 < kGalLinesMin)
         hipLaunchKernelGGL(k_gal_gather<16>, dim3(blocks_for(e1 - e0, 16)), dim3(256), 0, st, fine, E, ptr, src, e0,
                            e1, src_is_fine);
     else
-        return hipErrorInvalidValue;
+        hipLaunchKernelGGL(k_gal_gather_lines, dim3(blocks_for(e1 - e0, kGalEntries)), dim3(256), 0, st, fine, E, ptr,
+                           src, e0, e1, src_is_fine);
     MASX_CHECK_LAUNCH();
     return hipSuccess;
 }

@@ -11,9 +11,9 @@ bool   spmv_tiling_supported(int entries_per_thread);
 hipError_t launch_pack_values(const DevData& d, hipStream_t st);
 hipError_t launch_pack_abd(const DevData& d, const int* cp_body, const int* cp_sub, long long n_couplings,
                            float* vals_abd, hipStream_t st);
-// lanes per coarse entry: 16 or 64
+// long_lists: a wave per coarse entry
 hipError_t launch_gal_gather(const double* fine, double* E, const int* ptr, const int* src, int e0, int e1,
-                             int src_is_fine, int lanes, hipStream_t st);
+                             int src_is_fine, bool long_lists, hipStream_t st);
 // the map from stored position of a bank's inverse to its element (one
 // entry per stored value: FP32 floats or 16-bit halves), for the layout of
 // this bank size, precision and local kernel (DevData::mas_waves);

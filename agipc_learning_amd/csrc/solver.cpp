@@ -886,9 +886,8 @@ void Solver::build(int precision, hipStream_t user)
         // a whole wave per entry where the lists are long (the top levels)
         const int e0 = P.gal_level_ptr[g], e1 = P.gal_level_ptr[g + 1];
         const long long srcs = (long long)P.gal_level_src[g + 1] - P.gal_level_src[g];
-        const int lanes = srcs > 32ll * (e1 - e0) ? 64 : 16;
         MASX_HIP(launch_gal_gather(d_vals64_.ptr, d_E_.ptr, d_gal_ptr_.ptr, d_gal_src_.ptr, e0, e1,
-                                   P.gal_src_is_fine[g], lanes, aux));
+                                   P.gal_src_is_fine[g], srcs > 32ll * (e1 - e0), aux));
     }
     const int split = overlap ? P.n_fine_banks : P.n_banks;
     if(overlap)
