@@ -71,6 +71,7 @@ struct DevData
     const int* col;
     const int* entry_src;   // full entry -> upper block | transposed<<31
     const int* row_sys;
+    const int* i2e;         // internal row -> the caller's row, -1 padding
     // FP32 SpMV layout (tile-local symmetric pairs stored once; plan.hpp)
     const int* sy_row_ptr;  // n_rows+1
     const int* sy_col;      // column word: >= 0 outside the tile, else tile-local code

@@ -1157,20 +1157,6 @@ __global__ void __launch_bounds__(256) k_diag_factor(DevData d, const int* diag_
 
 // ================================================================ solve I/O
 
-__global__ void __launch_bounds__(256) k_load_rhs(DevData d, const int* ext_to_int, const double* b, int n_ext)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if(i >= n_ext) return;
-    const int R = ext_to_int[i];
-#pragma unroll
-    for(int c = 0; c < 3; ++c)
-    {
-        const double v = b[3 * (long long)i + c];
-        d.b64[3 * (long long)R + c] = v;
-        d.rt[3 * (long long)R + c]  = (float)v;
-    }
-}
-
 __global__ void __launch_bounds__(256) k_store_x(DevData d, const int* ext_to_int, double* x, int n_ext)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -2076,7 +2062,9 @@ __global__ void __launch_bounds__(256) k_mas_local_mfma(DevData d, int force)
 // result (MAS rows), 12x12 block-Jacobi (ABD bodies), identity or 3x3
 // block-Jacobi (plain rows); partial r.z.  The row data (and the coarse
 // corrections they need) are loaded while the r.r partials are reduced.
-__global__ void __launch_bounds__(256) k_precond_finish(DevData d, int force)
+// force (a preconditioner application on its own): whatever the systems'
+// states, z goes to the caller's FP64 rows z_ext if given.
+__global__ void __launch_bounds__(256) k_precond_finish(DevData d, int force, double* __restrict__ z_ext)
 {
     // rows by XCD as in the SpMV (each XCD a contiguous run of workgroups)
     const int wgi = xcd_tile(blockIdx.x, gridDim.x);
@@ -2189,7 +2177,13 @@ __global__ void __launch_bounds__(256) k_precond_finish(DevData d, int force)
             float acc = 0.f;
 #pragma unroll
             for(int j = 0; j < 12; ++j) acc += abd_p[j] * abd_r[j];
-            d.z[abd_base + abd_dof] = acc;
+            if(z_ext)
+            {
+                const int e = d.i2e[(int)(abd_base / 3) + abd_dof / 3];
+                if(e >= 0) z_ext[3 * (long long)e + abd_dof % 3] = (double)acc;
+            }
+            else
+                d.z[abd_base + abd_dof] = acc;
             part = (double)abd_r[abd_dof] * (double)acc;
         }
     }
@@ -2209,7 +2203,19 @@ __global__ void __launch_bounds__(256) k_precond_finish(DevData d, int force)
         {
             z0 = r0; z1 = r1; z2 = r2;
         }
-        d.z[o] = z0; d.z[o + 1] = z1; d.z[o + 2] = z2;
+        if(z_ext)
+        {
+            const int e = d.i2e[row];
+            if(e >= 0)
+            {
+                double* q = z_ext + 3 * (long long)e;
+                q[0] = (double)z0; q[1] = (double)z1; q[2] = (double)z2;
+            }
+        }
+        else
+        {
+            d.z[o] = z0; d.z[o + 1] = z1; d.z[o + 2] = z2;
+        }
         part = (double)r0 * z0 + (double)r1 * z1 + (double)r2 * z2;
     }
     if(force) return;
@@ -2642,7 +2648,10 @@ __global__ void __launch_bounds__(256) k_spmv_fused(DevData d, const float* __re
 // mode 1 (init / restart): r := rt.  Then the level-1 restriction of the MAS
 // rows and the partial r.r (b.b in FP64 at init).  The row vectors and the
 // component lists are loaded while the p.Ap partials are reduced.
-__global__ void __launch_bounds__(256) k_update(DevData d, const float* __restrict__ p, int mode)
+// mode 2 (a preconditioner application on its own): r := the caller's FP64
+// rows b_ext, whatever the systems' states.
+__global__ void __launch_bounds__(256) k_update(DevData d, const float* __restrict__ p, int mode,
+                                                const double* __restrict__ b_ext)
 {
     // rows by XCD as in the SpMV (each XCD a contiguous run of workgroups)
     const int wgi = xcd_tile(blockIdx.x, gridDim.x);
@@ -2679,7 +2688,7 @@ __global__ void __launch_bounds__(256) k_update(DevData d, const float* __restri
             return;
         }
     }
-    else
+    else if(mode == 1)
     {
         if(st.status != kRestarting && st.status != kInit) return;
         init = st.status == kInit;
@@ -2703,6 +2712,13 @@ __global__ void __launch_bounds__(256) k_update(DevData d, const float* __restri
             {
                 x[c] = d.x[o + c]; pv[c] = p[o + c]; rv[c] = d.r[o + c]; ap[c] = d.Ap[o + c];
             }
+        }
+        else if(mode == 2)
+        {
+            const int e = d.i2e[row];
+            if(e >= 0)
+#pragma unroll
+                for(int c = 0; c < 3; ++c) rv[c] = (float)b_ext[3 * (long long)e + c];
         }
         else
         {
@@ -3020,14 +3036,6 @@ __global__ void __launch_bounds__(256) k_spmv64(DevData d, const int* __restrict
     y[o] = a * acc + (b != 0.0 ? b * y[o] : 0.0);
 }
 
-__global__ void __launch_bounds__(256) k_z32_to_ext(const int* ext_to_int, const float* z, double* dst_ext, int n_ext)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if(i >= n_ext) return;
-    const long long R = ext_to_int[i];
-    for(int c = 0; c < 3; ++c) dst_ext[3 * (long long)i + c] = (double)z[3 * R + c];
-}
-
 // values[k] = src[indices[k]] for 9-double blocks (subsystem selection of
 // LocalPreconditioner::calculate_subsystem_bcoo_indices, i_preconditioner.cu:54-89)
 __global__ void __launch_bounds__(256) k_gather_blocks(const double* src, const uint32_t* idx, double* dst, long long n)
@@ -3214,14 +3222,6 @@ hipError_t launch_diag_factor(const DevData& d, const int* diag_src, const int* 
     return hipSuccess;
 }
 
-hipError_t launch_load_rhs(const DevData& d, const int* e2i, const double* b, int n_ext, hipStream_t st)
-{
-    if(n_ext <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_load_rhs, dim3(blocks_for(n_ext, 256)), dim3(256), 0, st, d, e2i, b, n_ext);
-    MASX_CHECK_LAUNCH();
-    return hipSuccess;
-}
-
 hipError_t launch_store_x(const DevData& d, const int* e2i, double* x, int n_ext, hipStream_t st)
 {
     if(n_ext <= 0) return hipSuccess;
@@ -3340,10 +3340,11 @@ hipError_t launch_mas_local(const DevData& d, int precision, int force, hipStrea
     return hipSuccess;
 }
 
-hipError_t launch_precond_finish(const DevData& d, int n_wg, int force, hipStream_t st, const LaunchEvents* ev)
+hipError_t launch_precond_finish(const DevData& d, int n_wg, int force, hipStream_t st, const LaunchEvents* ev,
+                                 double* z_ext)
 {
     if(n_wg <= 0) return hipSuccess;
-    MASX_DISPATCH(k_precond_finish, dim3(n_wg), dim3(256), d, force);
+    MASX_DISPATCH(k_precond_finish, dim3(n_wg), dim3(256), d, force, z_ext);
     MASX_CHECK_LAUNCH();
     return hipSuccess;
 }
@@ -3375,10 +3376,11 @@ hipError_t launch_spmv_fused(const DevData& d, int n_wg, int entries_per_thread,
     return hipSuccess;
 }
 
-hipError_t launch_update(const DevData& d, int n_wg, const float* p, int mode, hipStream_t st, const LaunchEvents* ev)
+hipError_t launch_update(const DevData& d, int n_wg, const float* p, int mode, hipStream_t st, const LaunchEvents* ev,
+                         const double* b_ext)
 {
     if(n_wg <= 0) return hipSuccess;
-    MASX_DISPATCH(k_update, dim3(n_wg), dim3(256), d, p, mode);
+    MASX_DISPATCH(k_update, dim3(n_wg), dim3(256), d, p, mode, b_ext);
     MASX_CHECK_LAUNCH();
     return hipSuccess;
 }
@@ -3408,14 +3410,6 @@ hipError_t launch_spmv64(const DevData& d, const int* i2e, const double* x, doub
 {
     if(d.n_rows == 0) return hipSuccess;
     hipLaunchKernelGGL(k_spmv64, dim3(blocks_for(d.n_rows, kRows64)), dim3(256), 0, st, d, i2e, x, a, b, y);
-    MASX_CHECK_LAUNCH();
-    return hipSuccess;
-}
-
-hipError_t launch_z32_to_ext(const int* e2i, const float* z, double* dst, int n_ext, hipStream_t st)
-{
-    if(n_ext <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_z32_to_ext, dim3(blocks_for(n_ext, 256)), dim3(256), 0, st, e2i, z, dst, n_ext);
     MASX_CHECK_LAUNCH();
     return hipSuccess;
 }

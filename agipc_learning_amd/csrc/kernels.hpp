@@ -26,7 +26,6 @@ hipError_t launch_mas_factor(const DevData& d, const double* E, const int* ent_p
                              int bank_end, hipStream_t st);
 hipError_t launch_abd_factor(const DevData& d, const int* body_src, float* inv, int n_bodies, hipStream_t st);
 hipError_t launch_diag_factor(const DevData& d, const int* diag_src, const int* needs, float* inv, hipStream_t st);
-hipError_t launch_load_rhs(const DevData& d, const int* e2i, const double* b, int n_ext, hipStream_t st);
 hipError_t launch_store_x(const DevData& d, const int* e2i, double* x, int n_ext, hipStream_t st);
 hipError_t launch_init_state(const DevData& d, int rule, double tol, const int* max_iter, int max_override,
                              int check_every, int frozen, hipStream_t st);
@@ -44,20 +43,21 @@ struct LaunchEvents
 };
 hipError_t launch_mas_local(const DevData& d, int precision, int force, hipStream_t st,
                             const LaunchEvents* ev = nullptr);
+// z_ext (with force): z as FP64 in the caller's rows instead of d.z
 hipError_t launch_precond_finish(const DevData& d, int n_wg, int force, hipStream_t st,
-                                 const LaunchEvents* ev = nullptr);
+                                 const LaunchEvents* ev = nullptr, double* z_ext = nullptr);
 // row-aligned tiles of at most 256 rows and 256 * entries_per_thread entries (2, 4 or 8)
 hipError_t launch_spmv_fused(const DevData& d, int n_wg, int entries_per_thread, const float* p_old, float* p_new,
                              hipStream_t st, const LaunchEvents* ev = nullptr);
+// mode 0: an iteration; 1: init / restart from d.rt; 2: r := b_ext (FP64, the caller's rows)
 hipError_t launch_update(const DevData& d, int n_wg, const float* p, int mode, hipStream_t st,
-                         const LaunchEvents* ev = nullptr);
+                         const LaunchEvents* ev = nullptr, const double* b_ext = nullptr);
 // true residual of the checked (or, report_only, all) systems and its decision
 hipError_t launch_true_residual(const DevData& d, int n_wg, int report_only, hipStream_t st);
 // rows of x in the internal order (zeros in padding rows), then y = a A x + b y for external rows
 hipError_t launch_rows_from_ext64(const int* i2e, const double* src, double* dst, int n_rows, hipStream_t st);
 hipError_t launch_spmv64(const DevData& d, const int* i2e, const double* x, double a, double b, double* y,
                          hipStream_t st);
-hipError_t launch_z32_to_ext(const int* e2i, const float* z, double* dst, int n_ext, hipStream_t st);
 hipError_t launch_gather_blocks(const double* src, const uint32_t* idx, double* dst, long long n, hipStream_t st);
 
 // Device arrays of doubles copied into one array by one launch: segment s,

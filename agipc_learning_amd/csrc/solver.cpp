@@ -650,6 +650,7 @@ void Solver::make_devdata()
     d.abd_cp_row = d_cp_row_.ptr;
     d.vals_abd = d_vals_abd_.ptr;
     d.row_sys = d_row_sys_.ptr;
+    d.i2e = d_i2e_.ptr;
     d.vals32 = d_vals32_.ptr;
     d.vals64 = d_vals64_.ptr;
     d.x = d_x_.ptr;
@@ -1063,16 +1064,11 @@ void Solver::apply_preconditioner(const double* d_r, double* d_z, hipStream_t us
 {
     if(!built_) throw std::runtime_error("build() must precede apply_preconditioner()");
     hipStream_t st = enter(user);
-    const size_t nvb = 3 * (size_t)plan_.n_rows * sizeof(float);
-    MASX_HIP(hipMemsetAsync(d_rt_.ptr, 0, nvb, st));
-    MASX_HIP(hipMemsetAsync(d_b64_.ptr, 0, 3 * (size_t)plan_.n_rows * sizeof(double), st));
-    MASX_HIP(launch_init_state(dd_, kRuleTrueRel, 0.0, d_max_iter_.ptr, 1, 0, 1, st));
-    MASX_HIP(launch_load_rhs(dd_, d_e2i_.ptr, d_r, plan_.n_ext, st));
-    MASX_HIP(launch_update(dd_, n_wg_upd_, d_p0_.ptr, 1, st));
-    MASX_HIP(launch_phase_finish(dd_, st));
+    // r from the caller's rows and its restriction, the local solves, the
+    // prolongation into the caller's rows
+    MASX_HIP(launch_update(dd_, n_wg_upd_, d_p0_.ptr, 2, st, nullptr, d_r));
     MASX_HIP(launch_mas_local(dd_, precision_, 1, st));
-    MASX_HIP(launch_precond_finish(dd_, n_wg_pre_, 1, st));
-    MASX_HIP(launch_z32_to_ext(d_e2i_.ptr, d_z_.ptr, d_z, plan_.n_ext, st));
+    MASX_HIP(launch_precond_finish(dd_, n_wg_pre_, 1, st, nullptr, d_z));
     leave(user);
 }
 
