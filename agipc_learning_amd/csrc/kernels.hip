@@ -3036,14 +3036,36 @@ __global__ void __launch_bounds__(256) k_spmv64(DevData d, const int* __restrict
     y[o] = a * acc + (b != 0.0 ? b * y[o] : 0.0);
 }
 
-// values[k] = src[indices[k]] for 9-double blocks (subsystem selection of
+// values[k] = src[indices[k]] (null: src[k]) for 9-double blocks (subsystem selection of
 // LocalPreconditioner::calculate_subsystem_bcoo_indices, i_preconditioner.cu:54-89)
 __global__ void __launch_bounds__(256) k_gather_blocks(const double* src, const uint32_t* idx, double* dst, long long n)
 {
     const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if(t >= 9 * n) return;
     const long long k = t / 9;
-    dst[t] = src[9 * (long long)idx[k] + t % 9];
+    dst[t] = src[9 * (idx ? (long long)idx[k] : k) + t % 9];
+}
+
+// *differs (host-visible, zero before) := 1 unless block k of the selection has
+// row rows[idx[k]] - offset == want_rows[k], column likewise (idx null: k), and
+// the pairs equal want_pairs.
+__global__ void __launch_bounds__(256) k_structure_differs(const int* __restrict__ rows, const int* __restrict__ cols,
+                                                           const uint32_t* __restrict__ idx, int offset, int n,
+                                                           const int* __restrict__ want_rows,
+                                                           const int* __restrict__ want_cols,
+                                                           const int* __restrict__ pairs,
+                                                           const int* __restrict__ want_pairs, int n_pair_ints,
+                                                           int* differs)
+{
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    bool bad = false;
+    if(t < n)
+    {
+        const uint32_t k = idx ? idx[t] : (uint32_t)t;
+        bad = rows[k] - offset != want_rows[t] || cols[k] - offset != want_cols[t];
+    }
+    if(t < n_pair_ints) bad |= pairs[t] != want_pairs[t];
+    if(bad) *(volatile int*)differs = 1;
 }
 
 // Up to kCopySegments device arrays of doubles copied into one array in a
@@ -3410,6 +3432,18 @@ hipError_t launch_spmv64(const DevData& d, const int* i2e, const double* x, doub
 {
     if(d.n_rows == 0) return hipSuccess;
     hipLaunchKernelGGL(k_spmv64, dim3(blocks_for(d.n_rows, kRows64)), dim3(256), 0, st, d, i2e, x, a, b, y);
+    MASX_CHECK_LAUNCH();
+    return hipSuccess;
+}
+
+hipError_t launch_structure_differs(const int* rows, const int* cols, const uint32_t* idx, int offset, int n,
+                                    const int* want_rows, const int* want_cols, const int* pairs,
+                                    const int* want_pairs, int n_pair_ints, int* differs, hipStream_t st)
+{
+    const int m = std::max(n, n_pair_ints);
+    if(m <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_structure_differs, dim3(blocks_for(m, 256)), dim3(256), 0, st, rows, cols, idx, offset, n,
+                       want_rows, want_cols, pairs, want_pairs, n_pair_ints, differs);
     MASX_CHECK_LAUNCH();
     return hipSuccess;
 }

@@ -17,6 +17,7 @@
 #include "hierarchy.hpp"
 #include "morton.hpp"
 #include "bandwidth.hpp"
+#include "kernels.hpp"
 #include "solver.hpp"
 
 namespace
@@ -85,14 +86,15 @@ struct masx_mas
     std::vector<uint32_t> nbr_list, nbr_start, nbr_num;
     std::vector<int>      part_to_real, real_to_part;
     bool uploaded = false, matrix_ready = false;
-    // structure of the last set_preconditioner_bcoo call
-    std::vector<int>      rows, cols, pairs;
+    // structure of the last set_preconditioner_bcoo call: block count, pair
+    // ints, and on the device its rows and columns (offset subtracted) and pairs
+    int n_blocks = -1, n_pair_ints = 0;
+    masx::DeviceArray<int> d_rows, d_cols, d_pairs;
     std::unique_ptr<masx_solver> solver;
-    uint32_t* d_sel = nullptr;  // selected block indices (device)
-    size_t    d_sel_n = 0;
+    int* h_differs = nullptr;  // coherent pinned: the structure comparison's answer
     ~masx_mas()
     {
-        if(d_sel) (void)hipFree(d_sel);
+        if(h_differs) (void)hipHostFree(h_differs);
     }
 };
 
@@ -768,104 +770,109 @@ int masx_mas_set_preconditioner_bcoo(masx_mas* m, const double* d_values, const 
     return guard([&] {
         require(m && m->matrix_ready, "init_matrix must come first");
         require(d_values && d_rows && d_cols && triplet_num >= 0, "bad matrix arguments");
+        require(cp_num >= 0, "negative pair count");
+        require(cp_num == 0 || d_pairs != nullptr, "null contact pairs");
         hipStream_t st = as_stream(stream);
-        // structure back to the host (the reference also synchronizes here:
-        // i_preconditioner.cu:83-86 and TraditionalMAS32Preconditioner.cu:2211)
-        std::vector<uint32_t> idx(triplet_num);
-        if(d_indices)
+        const int   n_pair_ints = 4 * cp_num;
+        // the structure of the call before, compared on the device: a Newton
+        // step that keeps it costs one flag instead of its download
+        bool same = m->solver && triplet_num == m->n_blocks && n_pair_ints == m->n_pair_ints;
+        if(same)
         {
-            if(triplet_num)
-                if(hipMemcpyAsync(idx.data(), d_indices, sizeof(uint32_t) * triplet_num, hipMemcpyDeviceToHost, st)
-                   != hipSuccess)
-                    throw std::runtime_error("index copy failed");
+            if(!m->h_differs) hip_ok(hipHostMalloc((void**)&m->h_differs, 64, hipHostMallocCoherent | hipHostMallocMapped));
+            int* d_differs = nullptr;
+            hip_ok(hipHostGetDevicePointer((void**)&d_differs, m->h_differs, 0));
+            *(volatile int*)m->h_differs = 0;
+            hip_ok(masx::launch_structure_differs(d_rows, d_cols, d_indices, offset, triplet_num, m->d_rows.ptr,
+                                                  m->d_cols.ptr, d_pairs, m->d_pairs.ptr, n_pair_ints, d_differs, st));
+            if(hipStreamSynchronize(st) != hipSuccess) throw std::runtime_error("stream sync failed");
+            same = *(volatile int*)m->h_differs == 0;
         }
-        else
-            for(int i = 0; i < triplet_num; ++i) idx[i] = (uint32_t)i;
-        if(hipStreamSynchronize(st) != hipSuccess) throw std::runtime_error("stream sync failed");
-        uint32_t max_idx = 0;
-        for(uint32_t v : idx) max_idx = std::max(max_idx, v);
-        const size_t n_all = triplet_num ? (size_t)max_idx + 1 : 0;
-        std::vector<int> all_r(n_all), all_c(n_all);
-        if(n_all)
+        if(!same)
         {
-            if(hipMemcpy(all_r.data(), d_rows, sizeof(int) * n_all, hipMemcpyDeviceToHost) != hipSuccess ||
-               hipMemcpy(all_c.data(), d_cols, sizeof(int) * n_all, hipMemcpyDeviceToHost) != hipSuccess)
-                throw std::runtime_error("structure copy failed");
-        }
-        std::vector<int> rows(triplet_num), cols(triplet_num), pairs(4 * (size_t)cp_num);
-        for(int i = 0; i < triplet_num; ++i)
-        {
-            rows[i] = all_r[idx[i]] - offset;
-            cols[i] = all_c[idx[i]] - offset;
-            require(rows[i] >= 0 && cols[i] >= 0 && rows[i] < m->vert_num && cols[i] < m->vert_num,
-                    "selected block outside the FEM range");
-        }
-        if(cp_num)
-        {
-            require(d_pairs != nullptr, "null contact pairs");
-            if(hipMemcpy(pairs.data(), d_pairs, sizeof(int) * 4 * cp_num, hipMemcpyDeviceToHost) != hipSuccess)
-                throw std::runtime_error("pair copy failed");
-        }
-        const bool same = m->solver && rows == m->rows && cols == m->cols && pairs == m->pairs;
-        if(!same && m->solver)
-        {
-            // a new structure on the same mesh (a new contact set): the solver
-            // keeps its topology and device buffers (ReorderRealtime runs again)
-            auto& d = m->solver->impl.system(0);
-            d.nb    = triplet_num;
-            d.rows  = rows;
-            d.cols  = cols;
-            d.pairs = pairs;
-            m->solver->impl.structure_changed(0);
-            m->solver->impl.setup();
-            m->rows  = std::move(rows);
-            m->cols  = std::move(cols);
-            m->pairs = std::move(pairs);
-        }
-        else if(!same)
-        {
-            m->solver = std::make_unique<masx_solver>();
-            masx::SystemDesc d;
-            d.block_rows   = m->vert_num;
-            d.nb           = triplet_num;
-            d.n_abd        = 0;
-            d.fem_offset   = 0;
-            d.n_fem        = m->vert_num;
-            d.use_mas      = true;
-            d.bank         = m->bank;
-            d.levels       = m->levels;
-            d.rows         = rows;
-            d.cols         = cols;
-            d.nbr_start    = m->nbr_start;
-            d.nbr_num      = m->nbr_num;
-            d.nbr_list     = m->nbr_list;
-            d.part_to_real = m->part_to_real;
-            d.real_to_part = m->real_to_part;
-            d.pairs        = pairs;
-            d.node_offset  = m->node_offset;
-            m->solver->impl.add_system(d);
-            m->solver->impl.setup();
-            m->rows  = std::move(rows);
-            m->cols  = std::move(cols);
-            m->pairs = std::move(pairs);
-            if(m->d_sel) (void)hipFree(m->d_sel);
-            m->d_sel   = nullptr;
-            m->d_sel_n = 0;
-        }
-        if(triplet_num)
-        {
-            if(m->d_sel_n < (size_t)triplet_num)
+            // structure back to the host (the reference also synchronizes here:
+            // i_preconditioner.cu:83-86 and TraditionalMAS32Preconditioner.cu:2211)
+            std::vector<uint32_t> idx(triplet_num);
+            if(d_indices)
             {
-                if(m->d_sel) (void)hipFree(m->d_sel);
-                if(hipMalloc((void**)&m->d_sel, sizeof(uint32_t) * triplet_num) != hipSuccess)
-                    throw std::runtime_error("allocation failed");
-                m->d_sel_n = triplet_num;
+                if(triplet_num)
+                    if(hipMemcpyAsync(idx.data(), d_indices, sizeof(uint32_t) * triplet_num, hipMemcpyDeviceToHost, st)
+                       != hipSuccess)
+                        throw std::runtime_error("index copy failed");
             }
-            // blocking copy: the gather below runs on the library's stream
-            if(hipMemcpy(m->d_sel, idx.data(), sizeof(uint32_t) * triplet_num, hipMemcpyHostToDevice) != hipSuccess)
-                throw std::runtime_error("index upload failed");
-            m->solver->impl.gather_values(0, d_values, m->d_sel, st);
+            else
+                for(int i = 0; i < triplet_num; ++i) idx[i] = (uint32_t)i;
+            if(hipStreamSynchronize(st) != hipSuccess) throw std::runtime_error("stream sync failed");
+            uint32_t max_idx = 0;
+            for(uint32_t v : idx) max_idx = std::max(max_idx, v);
+            const size_t n_all = triplet_num ? (size_t)max_idx + 1 : 0;
+            std::vector<int> all_r(n_all), all_c(n_all);
+            if(n_all)
+            {
+                if(hipMemcpy(all_r.data(), d_rows, sizeof(int) * n_all, hipMemcpyDeviceToHost) != hipSuccess ||
+                   hipMemcpy(all_c.data(), d_cols, sizeof(int) * n_all, hipMemcpyDeviceToHost) != hipSuccess)
+                    throw std::runtime_error("structure copy failed");
+            }
+            std::vector<int> rows(triplet_num), cols(triplet_num), pairs(n_pair_ints);
+            for(int i = 0; i < triplet_num; ++i)
+            {
+                rows[i] = all_r[idx[i]] - offset;
+                cols[i] = all_c[idx[i]] - offset;
+                require(rows[i] >= 0 && cols[i] >= 0 && rows[i] < m->vert_num && cols[i] < m->vert_num,
+                        "selected block outside the FEM range");
+            }
+            if(n_pair_ints)
+                if(hipMemcpy(pairs.data(), d_pairs, sizeof(int) * n_pair_ints, hipMemcpyDeviceToHost) != hipSuccess)
+                    throw std::runtime_error("pair copy failed");
+            m->n_blocks = -1;  // until the new structure is set up
+            if(m->solver)
+            {
+                // a new structure on the same mesh (a new contact set): the solver
+                // keeps its topology and device buffers (ReorderRealtime runs again)
+                auto& d = m->solver->impl.system(0);
+                d.nb    = triplet_num;
+                d.rows  = rows;
+                d.cols  = cols;
+                d.pairs = pairs;
+                m->solver->impl.structure_changed(0);
+                m->solver->impl.setup();
+            }
+            else
+            {
+                auto solver = std::make_unique<masx_solver>();
+                masx::SystemDesc d;
+                d.block_rows   = m->vert_num;
+                d.nb           = triplet_num;
+                d.n_abd        = 0;
+                d.fem_offset   = 0;
+                d.n_fem        = m->vert_num;
+                d.use_mas      = true;
+                d.bank         = m->bank;
+                d.levels       = m->levels;
+                d.rows         = rows;
+                d.cols         = cols;
+                d.nbr_start    = m->nbr_start;
+                d.nbr_num      = m->nbr_num;
+                d.nbr_list     = m->nbr_list;
+                d.part_to_real = m->part_to_real;
+                d.real_to_part = m->real_to_part;
+                d.pairs        = pairs;
+                d.node_offset  = m->node_offset;
+                solver->impl.add_system(d);
+                solver->impl.setup();
+                m->solver = std::move(solver);
+            }
+            auto keep = [](masx::DeviceArray<int>& a, const std::vector<int>& h) {
+                a.alloc(h.size());
+                if(!h.empty()) hip_ok(hipMemcpy(a.ptr, h.data(), h.size() * sizeof(int), hipMemcpyHostToDevice));
+            };
+            keep(m->d_rows, rows);
+            keep(m->d_cols, cols);
+            keep(m->d_pairs, pairs);
+            m->n_blocks    = triplet_num;
+            m->n_pair_ints = n_pair_ints;
         }
+        if(triplet_num) m->solver->impl.gather_values(0, d_values, d_indices, st);
         m->solver->impl.build(precision, st);
         if(hipStreamSynchronize(st) != hipSuccess) throw std::runtime_error("build failed");
     });

@@ -140,3 +140,46 @@ def test_lane_tiles_agree_with_the_block_diagonal_layout(bank, precision, n, con
         b = dev(session.rhs_of(w))
         st = s.solve(b, torch.zeros_like(b), max_iter=200)[0]
         assert st["failure"] == 0 and st["rel_res_true"] <= 1e-4 * (1 + 1e-6)
+
+
+def test_mas_object_sees_a_structure_of_the_same_size():
+    """A call with as many blocks and pairs as the last but another order of
+    blocks, or other pairs, is not taken for the same structure: its apply
+    equals a fresh object's bit for bit.  The selection may be null."""
+    from agipc_learning_amd import workloads as W
+
+    w = W.fem_grid(9, n_contacts=120, seed=4, young_sigma=0.5)
+    nv, nb = w["n_vertices"], len(w["rows"])
+    p2r, r2p = native.morton_partition(w["positions"])
+    start, num, lst = W.neighbors(nv, w["tets"])
+    rng = np.random.default_rng(8)
+    R = dev(rng.standard_normal(3 * nv))
+
+    def fresh():
+        m = native.MasPreconditioner(32)
+        m.init_neighbor(nv, 0, len(lst), len(p2r))
+        m.upload(lst, start, num, p2r, r2p)
+        m.init_matrix()
+        return m
+
+    def apply(m, order, pairs, select=True):
+        idx = dev(order.astype(np.int32)) if select else None
+        vals, rows, cols = (w["vals"], w["rows"], w["cols"]) if select else (w["vals"][order], w["rows"][order], w["cols"][order])
+        p = dev(np.ascontiguousarray(pairs, np.int32))
+        m.set_preconditioner_bcoo(dev(vals), dev(rows), dev(cols), idx, 0, nb, pairs=p, cp_num=len(pairs))
+        Z = torch.zeros_like(R)
+        m.preconditioning(R, Z)
+        return host(Z)
+
+    plain, mixed = np.arange(nb), rng.permutation(nb)
+    other = np.roll(np.asarray(w["pairs"]).reshape(-1, 4), 7, axis=1)
+    other = (other + 13) % nv
+    m = fresh()
+    steps = [(plain, w["pairs"], True), (mixed, w["pairs"], True), (mixed, w["pairs"], False), (mixed, other, True),
+             (plain, w["pairs"], True)]
+    for order, pairs, select in steps:
+        for _ in range(2):  # the second call keeps the structure
+            assert np.array_equal(apply(m, order, pairs, select), apply(fresh(), order, pairs, select))
+    with pytest.raises(RuntimeError):
+        m.set_preconditioner_bcoo(dev(w["vals"]), dev(w["rows"]), dev(w["cols"]), dev(plain.astype(np.int32)), 1, nb,
+                                  pairs=dev(np.asarray(w["pairs"], np.int32)), cp_num=len(w["pairs"]))
