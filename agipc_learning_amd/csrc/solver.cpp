@@ -974,7 +974,6 @@ void Solver::solve(const double* d_b, double* d_x, const SolveParams& prm, std::
     const int max_chunks = max_total / chunk + 8 + (with_check ? max_total / 10 : 0);
     // Chunks are launched ahead of the status checks: kDepth in flight, and
     // up to 80% of the previous solve's iterations before the first check.
-    // A chunk launched after convergence costs only its early-exit launches.
     const size_t state_bytes = sizeof(SysState) * P.n_sys;
     // Every chunk ends by writing (unfinished count, sequence number) to host
     // memory; the host polls that instead of a per-chunk event or copy.
@@ -1006,11 +1005,19 @@ void Solver::solve(const double* d_b, double* d_x, const SolveParams& prm, std::
         }
     };
     const int ahead = std::min(max_chunks, std::max(kDepth, (int)(0.8 * last_iters_) / chunk));
+    // The previous solve's iterations predict where this one ends: there (and
+    // one chunk later) the next chunk waits for the status of the one before.
+    // A chunk launched past convergence is ~30 launches that exit at once,
+    // 50-60 us before the result can be read (8^3 grid, FP32, 40 iterations:
+    // 1225 -> 1168 us a solve with its build); a wait costs ~10 us when the solve goes
+    // on.  Further on the prediction has failed and chunks go out ahead again.
+    const int needed = last_iters_ > 0 ? last_iters_ / chunk + 1 : max_chunks;
+    auto      depth  = [&] { return launched >= needed && launched < needed + 2 ? 1 : kDepth; };
     while(launched < ahead) launch_one();
     checked = std::max(0, launched - kDepth);
     for(;;)
     {
-        while(launched < max_chunks && launched - checked < kDepth) launch_one();
+        while(launched < max_chunks && launched - checked < depth()) launch_one();
         if(checked >= launched) break;
         // a later chunk may already have overwritten the count, which only moves it on
         wait_export(seq0 + checked + 1);
