@@ -135,6 +135,11 @@ __global__ void k_dp_gal_items(int lvl, long long n, const int* rows, const int*
                                const int* ES, int e_prev, DpSystems sys, const int* gn_all, const int* lvl_begin,
                                int bits, uint64_t* keys, int* vals, int* n_valid)
 {
+    // valid items are counted in LDS: a global add per thread made every wave
+    // queue at one address (34 us a level on 0.6 million items)
+    __shared__ int s_valid;
+    if(threadIdx.x == 0) s_valid = 0;
+    __syncthreads();
     int valid = 0;
     for(long long k = blockIdx.x * (long long)blockDim.x + threadIdx.x; k < n; k += (long long)gridDim.x * blockDim.x)
     {
@@ -173,7 +178,9 @@ __global__ void k_dp_gal_items(int lvl, long long n, const int* rows, const int*
         vals[k] = src << 2 | mode;
         ++valid;
     }
-    if(valid) atomicAdd(n_valid, valid);
+    if(valid) atomicAdd(&s_valid, valid);
+    __syncthreads();
+    if(threadIdx.x == 0 && s_valid) atomicAdd(n_valid, s_valid);
 }
 
 __global__ void k_dp_run_ends(long long n, const uint64_t* keys, int* flag)
@@ -242,27 +249,48 @@ __device__ __forceinline__ int coarse_bank_of(const DpSystems& sys, int n_fine_b
     return n_fine_banks + (sys.coarse_base[s] + I - sys.n_slots[s]) / bank;
 }
 
+// Coarse entries are sorted by their row node within a level, so the lanes of
+// a wave hold runs of entries whose rows lie in one bank: one atomic a run (one
+// an entry queued at the bank's counter: 41 us each on a 40^3 grid's levels).
+// The lanes of this lane's run, all of them active.
+__device__ __forceinline__ unsigned long long bank_run(int gb)
+{
+    const int lane = (int)threadIdx.x & 63;
+    const int before = __shfl_up(gb, 1);
+    const unsigned long long heads = __ballot(lane == 0 || before != gb);
+    const unsigned long long upto = heads & (~0ull >> (63 - lane));       // heads at or before this lane
+    const int first = 63 - __clzll((long long)upto);                      // lane 0 is a head
+    const unsigned long long after = lane == 63 ? 0 : heads >> (lane + 1);
+    const int last = after ? lane + __ffsll((long long)after) - 1 : 63;
+    return (~0ull >> (63 - last)) & (~0ull << first);
+}
+
 __global__ void k_dp_ent_flag_coarse(int n_gal, int bank, int n_fine_banks, DpSystems sys, const int* EI, const int* EJ,
                                      const int* ES, int* flag, int* bank_cnt)
 {
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if(e > n_gal) return;
-    int f = 0;
+    int f = 0, gb = -1;
     if(e < n_gal)
     {
         const int I = EI[e], J = EJ[e];
-        f = I / bank == J / bank;
-        if(f) atomicAdd(&bank_cnt[coarse_bank_of(sys, n_fine_banks, bank, ES[e], I)], 1);
+        f  = I / bank == J / bank;
+        gb = coarse_bank_of(sys, n_fine_banks, bank, ES[e], I);
     }
-    flag[e] = f;
+    const unsigned long long in_run = __ballot(f) & bank_run(gb);  // the run's entries inside the bank
+    if(f && __ffsll((long long)in_run) - 1 == ((int)threadIdx.x & 63)) atomicAdd(&bank_cnt[gb], __popcll(in_run));
+    if(e <= n_gal) flag[e] = f;
 }
 
 __global__ void k_dp_ent_first_coarse(int n_gal, int bank, int n_fine_banks, DpSystems sys, const int* EI,
                                       const int* ES, const int* flag, const int* fpos, int* bank_first)
 {
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if(e >= n_gal || !flag[e]) return;
-    atomicMin(&bank_first[coarse_bank_of(sys, n_fine_banks, bank, ES[e], EI[e])], fpos[e]);
+    const bool in = e < n_gal;
+    const int  f  = in ? flag[e] : 0;
+    const int  gb = in ? coarse_bank_of(sys, n_fine_banks, bank, ES[e], EI[e]) : -1;
+    const unsigned long long in_run = __ballot(f) & bank_run(gb);
+    // fpos grows with e: the run's first entry holds its smallest
+    if(f && __ffsll((long long)in_run) - 1 == ((int)threadIdx.x & 63)) atomicMin(&bank_first[gb], fpos[e]);
 }
 
 __global__ void k_dp_ent_fill_coarse(int n_gal, int bank, int n_fine_banks, DpSystems sys, const int* EI,
@@ -284,31 +312,40 @@ __global__ void k_dp_ent_bank_counts(int n_fine_banks, int bank, const int* row_
 }
 
 // the greedy tile that starts at r0 (build_spmv_layout's cut, from any r0).
-// A workgroup takes kThreads consecutive r0, whose tiles can only reach the
-// next kThreads + kSpmvTileRows - 1 rows: their row pointers, and their
-// column words when they fit kSlCols, are staged in LDS once, so each
-// thread's per-row searches (two per row it adds) read LDS instead of HBM.
-constexpr int kSlRows = kThreads + kSpmvTileRows;
-constexpr int kSlCols = 8192;
+// Bound by the chain of row searches behind one start: a thread that adds its
+// rows one by one makes ~100 dependent ones (165 us on 88,922 rows).  Here a
+// wave takes a start, its lanes 64 rows at a time: each lane finds what its row
+// adds, a prefix sum finds the row that no longer fits.  A workgroup takes
+// kSlStarts consecutive starts, whose tiles can only reach the next
+// kSlStarts + kSpmvTileRows - 1 rows: their row pointers, the place of their
+// diagonals and, when they fit kSlCols, their columns are staged in LDS.
+constexpr int kSlStarts  = 128;
+constexpr int kSlRows    = kSlStarts + kSpmvTileRows;
+constexpr int kSlCols    = 12288;
+constexpr int kSlThreads = 1024;
 
-__global__ void __launch_bounds__(kThreads) k_dp_sl_next(int n, const int* row_ptr, const int* col, const int* row_sys,
-                                                         const int* row_off, int cap, int* nxt, int* kept)
+__global__ void __launch_bounds__(kSlThreads) k_dp_sl_next(int n, const int* row_ptr, const int* col,
+                                                           const int* row_sys, const int* row_off, int cap, int* nxt,
+                                                           int* kept)
 {
     __shared__ int s_ptr[kSlRows + 1];
+    __shared__ int s_diag[kSlRows];
+    __shared__ int s_end[kSlStarts];
     __shared__ int s_col[kSlCols];
-    const int R = blockIdx.x * kThreads, r0 = R + (int)threadIdx.x;
+    const int R = blockIdx.x * kSlStarts;
     const int rw = min(n, R + kSlRows);  // rows [R, rw) are staged
-    for(int i = threadIdx.x; i <= rw - R; i += kThreads) s_ptr[i] = row_ptr[R + i];
+    for(int i = threadIdx.x; i <= rw - R; i += kSlThreads) s_ptr[i] = row_ptr[R + i];
+    // a tile ends at its system's end or at kSpmvTileRows
+    for(int i = threadIdx.x; i < min(kSlStarts, n - R); i += kSlThreads)
+        s_end[i] = min(row_off[row_sys[R + i] + 1], R + i + kSpmvTileRows);
     __syncthreads();
     const int e0 = s_ptr[0], ne = s_ptr[rw - R] - e0;
     const bool cached = ne <= kSlCols;  // uniform
     if(cached)
-        for(int i = threadIdx.x; i < ne; i += kThreads) s_col[i] = col[e0 + i];
+        for(int i = threadIdx.x; i < ne; i += kSlThreads) s_col[i] = col[e0 + i];
     __syncthreads();
-    if(r0 >= n) return;
-    // first entry of row r (R <= r < rw) whose column is >= c
-    auto first_ge_s = [&](int r, int c) {
-        int lo = s_ptr[r - R], hi = s_ptr[r + 1 - R];
+    // first entry in [lo, hi) whose column is >= c
+    auto first_ge_s = [&](int lo, int hi, int c) {
         while(lo < hi)
         {
             const int mid = (lo + hi) >> 1;
@@ -319,27 +356,61 @@ __global__ void __launch_bounds__(kThreads) k_dp_sl_next(int n, const int* row_p
         }
         return lo;
     };
-    const int r_end = row_off[row_sys[r0] + 1];  // the system's end
-    int k = s_ptr[r0 + 1 - R] - s_ptr[r0 - R];
-    int r1 = r0 + 1;
-    while(r1 < r_end && r1 - r0 < kSpmvTileRows)
+    for(int i = threadIdx.x; i < rw - R; i += kSlThreads) s_diag[i] = first_ge_s(s_ptr[i], s_ptr[i + 1], R + i);
+    __syncthreads();
+    const int lane = (int)threadIdx.x & 63;
+    for(int r0 = R + (int)threadIdx.x / 64; r0 < min(n, R + kSlStarts); r0 += kSlThreads / 64)  // uniform in a wave
     {
-        // r1 + 1 <= r0 + kSpmvTileRows <= R + kSlRows - 1 and r1 < n: inside the staged rows
-        const int q = (s_ptr[r1 + 1 - R] - first_ge_s(r1, r1)) + (first_ge_s(r1, r0) - s_ptr[r1 - R]);
-        if(k + q > cap) break;
-        k += q;
-        ++r1;
+        const int r_end = s_end[r0 - R];
+        int k = s_ptr[r0 + 1 - R] - s_ptr[r0 - R];
+        int r1 = r0 + 1;
+        while(r1 < r_end)
+        {
+            // r < r_end <= min(n, R + kSlRows - 1): inside the staged rows
+            const int r = r1 + lane;
+            int q = 0;
+            if(r < r_end)
+                q = (s_ptr[r + 1 - R] - s_diag[r - R]) + (first_ge_s(s_ptr[r - R], s_diag[r - R], r0) - s_ptr[r - R]);
+            int sum = q;
+#pragma unroll
+            for(int d = 1; d < 64; d <<= 1)
+            {
+                const int o = __shfl_up(sum, d);
+                if(lane >= d) sum += o;
+            }
+            const unsigned long long stop = __ballot(r >= r_end || k + sum > cap);
+            if(stop)
+            {
+                const int f = __ffsll((long long)stop) - 1;  // the first row that is not added
+                if(f > 0) k += __shfl(sum, f - 1);
+                r1 += f;
+                break;
+            }
+            k += __shfl(sum, 63);
+            r1 += 64;
+        }
+        if(lane == 0)
+        {
+            nxt[r0]  = r1;
+            kept[r0] = k;
+        }
     }
-    nxt[r0]  = r1;
-    kept[r0] = k;
 }
 
-// The chain of tiles from row 0, walked by one thread through windows of the
-// tile ends staged in LDS (each step r -> nxt[r] advances by 1..256 rows).
-constexpr int kChainWindow = 32768;
+// The chain of tiles from row 0, one workgroup, in windows of the tile ends
+// staged in LDS (each step r -> nxt[r] advances by 1..256 rows).  One thread
+// walking the window is a chain of ~300 LDS reads (63 us on 88,922 rows), so
+// the window is cut into segments: for each of the 256 rows where the chain
+// can enter one, a thread walks it to its end; one thread then links the
+// segments, and a thread per segment writes its tiles.
+constexpr int kChainWindow   = 32768;
+constexpr int kChainSegment  = 2048;  // longer than a step
+constexpr int kChainSegments = kChainWindow / kChainSegment;
 __global__ void __launch_bounds__(1024) k_dp_sl_chain(int n, const int* nxt, int* ts, int* n_tiles)
 {
     __shared__ unsigned char step[kChainWindow];
+    __shared__ int walk[kChainSegments * kSpmvTileRows];  // [segment][entry]: tiles << 8 | rows past the end
+    __shared__ int s_entry[kChainSegments], s_first[kChainSegments];
     __shared__ int s_r, s_t;
     if(threadIdx.x == 0)
     {
@@ -352,18 +423,42 @@ __global__ void __launch_bounds__(1024) k_dp_sl_chain(int n, const int* nxt, int
         const int w0 = s_r;
         if(w0 >= n) break;  // uniform: every thread read the same s_r
         const int wn = min(kChainWindow, n - w0);
-        for(int i = threadIdx.x; i < wn; i += blockDim.x) step[i] = (unsigned char)(nxt[w0 + i] - (w0 + i) - 1);
+        const int ns = (wn + kChainSegment - 1) / kChainSegment;
+#pragma unroll 8
+        for(int i = threadIdx.x; i < wn; i += 1024) step[i] = (unsigned char)(nxt[w0 + i] - (w0 + i) - 1);
+        __syncthreads();
+        for(int i = threadIdx.x; i < ns * kSpmvTileRows; i += 1024)
+        {
+            const int g = i / kSpmvTileRows, end = min(wn, (g + 1) * kChainSegment);
+            int r = g * kChainSegment + i % kSpmvTileRows, t = 0;
+            while(r < end)
+            {
+                r += step[r] + 1;
+                ++t;
+            }
+            walk[i] = t << 8 | ((r - end) & 255);  // r - end <= 255 wherever the chain enters
+        }
         __syncthreads();
         if(threadIdx.x == 0)
         {
-            int r = w0, t = s_t;
-            while(r < w0 + wn)
+            int entry = 0, t = s_t;
+            for(int g = 0; g < ns; ++g)
             {
-                ts[t++] = r;
-                r += step[r - w0] + 1;
+                s_entry[g] = entry;
+                s_first[g] = t;
+                const int w = walk[g * kSpmvTileRows + entry];
+                t += w >> 8;
+                entry = w & 255;
             }
-            s_r = r;
+            s_r = w0 + wn + entry;
             s_t = t;
+        }
+        __syncthreads();
+        if((int)threadIdx.x < ns)
+        {
+            const int g = (int)threadIdx.x, end = min(wn, (g + 1) * kChainSegment);
+            int t = s_first[g];
+            for(int r = g * kChainSegment + s_entry[g]; r < end; r += step[r] + 1) ts[t++] = w0 + r;
         }
     }
     if(threadIdx.x == 0) *n_tiles = s_t;
@@ -394,6 +489,13 @@ __global__ void __launch_bounds__(kThreads) k_dp_sl_tile_counts(int n_tiles, int
     }
 }
 
+// One tile's words.  Eight lanes take a row; a row's entries before the tile's
+// first column (s_below) and from its diagonal on (s_diag) are kept, so an
+// entry's place follows from its own index.  Columns are searched in LDS when
+// the tile's fit kFillCols (a thread per row walking and searching in global
+// memory: 75 us on 88,922 rows).
+constexpr int kFillCols = 6144;
+
 __global__ void __launch_bounds__(kThreads) k_dp_sl_fill(int n_tiles, int n, const int* ts, const int* kept,
                                                          const int* e_base, const int* q_base, const int* row_ptr,
                                                          const int* col, const int* entry_src, const int* row_sys,
@@ -401,47 +503,72 @@ __global__ void __launch_bounds__(kThreads) k_dp_sl_fill(int n_tiles, int n, con
                                                          int2* wg_ent, int* err)
 {
     __shared__ int s_scan[kThreads];
-    __shared__ int s_tstart[kThreads + 1];
+    __shared__ int s_tstart[kThreads], s_ptr[kThreads + 1], s_below[kThreads], s_diag[kThreads], s_out[kThreads];
+    __shared__ int s_col[kFillCols];
     const int t = blockIdx.x;
     const int r0 = ts[t], r1 = t + 1 < n_tiles ? ts[t + 1] : n, nr = r1 - r0;
     const int j = (int)threadIdx.x, r = r0 + j;
+    const int x0 = row_ptr[r0], nx = row_ptr[r1] - x0;
+    const bool cached = nx <= kFillCols;  // uniform
+    for(int i = j; i <= nr; i += kThreads) s_ptr[i] = row_ptr[r0 + i];
+    if(cached)
+        for(int i = j; i < nx; i += kThreads) s_col[i] = col[x0 + i];
+    __syncthreads();
+    auto col_at = [&](int e) { return cached ? s_col[e - x0] : col[e]; };
+    auto first_ge_s = [&](int lo, int hi, int c) {  // first entry in [lo, hi) whose column is >= c
+        while(lo < hi)
+        {
+            const int mid = (lo + hi) >> 1;
+            if(col_at(mid) < c)
+                lo = mid + 1;
+            else
+                hi = mid;
+        }
+        return lo;
+    };
     int cnt = 0, kr = 0;
     if(j < nr)
     {
-        const int d = first_ge(row_ptr, col, r, r), b = first_ge(row_ptr, col, r, r0);
-        cnt = d - b;                                    // entries (r', r), r0 <= r' < r: by symmetry
-        kr  = (row_ptr[r + 1] - d) + (b - row_ptr[r]);  // entries row r keeps
+        const int d = first_ge_s(s_ptr[j], s_ptr[j + 1], r), b = first_ge_s(s_ptr[j], d, r0);
+        cnt = d - b;                                  // entries (r', r), r0 <= r' < r: by symmetry
+        kr  = (s_ptr[j + 1] - d) + (b - s_ptr[j]);    // entries row r keeps
+        s_diag[j]  = d;
+        s_below[j] = b;
     }
     int n_trans, n_kept;
     const int tst  = block_exclusive_scan(cnt, s_scan, &n_trans);
     const int koff = block_exclusive_scan(kr, s_scan, &n_kept);
     s_tstart[j] = tst;
-    if(j == 0) s_tstart[kThreads] = n_trans;
+    s_out[j]    = e_base[t] + koff;
     __syncthreads();
     if(j == 0 && n_trans > kSpmvMaxCap) atomicOr(err, 4);
-    if(j < nr && n_trans <= kSpmvMaxCap)
+    if(n_trans <= kSpmvMaxCap)
     {
-        int o = e_base[t] + koff;
-        L_row_ptr[r] = o;
-        L_tptr[r]    = q_base[t] + tst;
-        unsigned first = kSpmvRowStart;
-        for(int e = row_ptr[r]; e < row_ptr[r + 1]; ++e)
+        if(j < nr)
         {
-            const int c = col[e];
-            unsigned word = (unsigned)c;
-            if(c >= r0 && c < r1)
+            L_row_ptr[r] = s_out[j];
+            L_tptr[r]    = q_base[t] + tst;
+        }
+        for(int w = j / 8; w < nr; w += kThreads / 8)
+        {
+            const int rr = r0 + w, p = s_ptr[w], b = s_below[w], d = s_diag[w];
+            for(int e = p + j % 8; e < s_ptr[w + 1]; e += 8)
             {
-                if(c < r) continue;  // the tile's lower copy: its upper twin covers it
-                const int tpos = c == r ? 0
-                                        : s_tstart[c - r0] +
-                                              (first_ge(row_ptr, col, c, r) - first_ge(row_ptr, col, c, r0)) +
-                                              (e - first_ge(row_ptr, col, r, c));
-                word = kSpmvInTile | (unsigned)tpos << 16 | (unsigned)(r - r0) << 8 | (unsigned)(c - r0);
+                if(e >= b && e < d) continue;  // the tile's lower copy: its upper twin covers it
+                const int c = col_at(e), at = e < b ? e - p : e - d + (b - p);
+                unsigned word = (unsigned)c;
+                if(e >= d && c < r1)
+                {
+                    const int k = c - r0;
+                    const int tpos = c == rr ? 0
+                                             : s_tstart[k] + (first_ge_s(s_below[k], s_diag[k], rr) - s_below[k]) +
+                                                   (e - first_ge_s(d, e, c));
+                    word = kSpmvInTile | (unsigned)tpos << 16 | (unsigned)w << 8 | (unsigned)k;
+                }
+                if(at == 0) word |= kSpmvRowStart;
+                L_col[s_out[w] + at] = (int)word;
+                L_src[s_out[w] + at] = entry_src[e];
             }
-            L_col[o] = (int)(word | first);
-            L_src[o] = entry_src[e];
-            first = 0;
-            ++o;
         }
     }
     if(j == 0)
@@ -602,7 +729,7 @@ hipError_t dp_sl_next(int n, const int* row_ptr, const int* col, const int* row_
                       int* nxt, int* kept, hipStream_t st)
 {
     if(n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_dp_sl_next, dim3((n + kThreads - 1) / kThreads), dim3(kThreads), 0, st, n, row_ptr, col,
+    hipLaunchKernelGGL(k_dp_sl_next, dim3((n + kSlStarts - 1) / kSlStarts), dim3(kSlThreads), 0, st, n, row_ptr, col,
                        row_sys, row_off, cap, nxt, kept);
     return hipGetLastError();
 }

@@ -183,3 +183,31 @@ def test_mas_object_sees_a_structure_of_the_same_size():
     with pytest.raises(RuntimeError):
         m.set_preconditioner_bcoo(dev(w["vals"]), dev(w["rows"]), dev(w["cols"]), dev(plain.astype(np.int32)), 1, nb,
                                   pairs=dev(np.asarray(w["pairs"], np.int32)), cp_num=len(w["pairs"]))
+
+
+@pytest.mark.parametrize("sizes,per_row,hub", [((1,), 0, 0), ((256, 257), 0, 0), ((33100, 40), 0, 0), ((129, 127), 2, 90),
+                                               ((700,), 24, 600), ((35000,), 2, 300)])
+def test_device_structure_around_tile_ends(sizes, per_row, hub):
+    """The device's SpMV tiles, entry lists and Galerkin maps equal the host's:
+    tiles that end at 256 rows, at a system's end and at the entry cap, a chain
+    of tiles longer than one staged window and than one of its segments, rows
+    whose columns do not fit the staged ones, and a row of more than a tile."""
+    rng = np.random.default_rng(sum(sizes) + hub)
+    systems = [(n,) + random_structure(n, per_row, min(hub, n), rng) + (rng.random((n, 3)),) for n in sizes]
+    solvers = []
+    for on_device in (0, 1):
+        s = native.Solver()
+        for n, rows, cols, pos in systems:
+            i = s.add_system(block_rows=n, rows=rows, cols=cols)
+            s.set_topology_morton(i, np.zeros(n), np.zeros(n), [], pos)
+        if not on_device:
+            s.set_device_structure(0)
+        s.setup()
+        assert s.device_structure_used() == bool(on_device)
+        solvers.append(s)
+    want, got = solvers
+    for entries in (2, 4, 8):
+        for s in solvers:
+            s.set_spmv_tiling(entries)
+        for name in native.Solver.PLAN_ARRAYS:
+            assert np.array_equal(want.plan_array(name), got.plan_array(name)), (entries, name)
