@@ -83,7 +83,7 @@ __global__ void k_dp_fill(int* p, int value, long long n)
 }
 
 __global__ void k_dp_csr_items(long long nb, const int* rows, const int* cols, DpSystems sys, const int* e2i,
-                               int n_rows, int bits, uint64_t* keys, int* vals, int* row_cnt, int* diag_src, int* err)
+                               int n_rows, int bits, uint64_t* keys, int* vals, int* diag_src, int* err)
 {
     const uint64_t sentinel = (uint64_t)n_rows << bits;
     for(long long k = blockIdx.x * (long long)blockDim.x + threadIdx.x; k < nb; k += (long long)gridDim.x * blockDim.x)
@@ -105,7 +105,6 @@ __global__ void k_dp_csr_items(long long nb, const int* rows, const int* cols, D
             vals[2 * k]     = (int)k;
             keys[2 * k + 1] = sentinel;
             vals[2 * k + 1] = -1;
-            atomicAdd(&row_cnt[iR], 1);
             atomicMax(&diag_src[iR], (int)k);  // the last diagonal block of the row
         }
         else
@@ -115,9 +114,19 @@ __global__ void k_dp_csr_items(long long nb, const int* rows, const int* cols, D
             vals[2 * k]     = (int)k;
             keys[2 * k + 1] = (uint64_t)iC << bits | (uint64_t)iR;
             vals[2 * k + 1] = (int)k | (int)0x80000000u;
-            atomicAdd(&row_cnt[iR], 1);
-            atomicAdd(&row_cnt[iC], 1);
         }
+    }
+}
+
+// row_ptr from the sorted items: row r starts at the first item of a row >= r.
+// The starts fall out of the sort; counting them as the items are made took an
+// atomic an item (46 us for 590,000 blocks, 17 without) and a scan.
+__global__ void k_dp_row_starts(long long n, const uint64_t* keys, int bits, int n_rows, int* row_ptr)
+{
+    for(long long x = blockIdx.x * (long long)blockDim.x + threadIdx.x; x <= n; x += (long long)gridDim.x * blockDim.x)
+    {
+        const int r = x < n ? (int)(keys[x] >> bits) : n_rows;
+        for(int q = x > 0 ? (int)(keys[x - 1] >> bits) + 1 : 0; q <= r; ++q) row_ptr[q] = (int)x;
     }
 }
 
@@ -136,7 +145,8 @@ __global__ void k_dp_gal_items(int lvl, long long n, const int* rows, const int*
                                int bits, uint64_t* keys, int* vals, int* n_valid)
 {
     // valid items are counted in LDS: a global add per thread made every wave
-    // queue at one address (34 us a level on 0.6 million items)
+    // queue at one address (34 us a level from 0.6 million items, 9 now
+    // with four items a thread)
     __shared__ int s_valid;
     if(threadIdx.x == 0) s_valid = 0;
     __syncthreads();
@@ -251,7 +261,7 @@ __device__ __forceinline__ int coarse_bank_of(const DpSystems& sys, int n_fine_b
 
 // Coarse entries are sorted by their row node within a level, so the lanes of
 // a wave hold runs of entries whose rows lie in one bank: one atomic a run (one
-// an entry queued at the bank's counter: 41 us each on a 40^3 grid's levels).
+// an entry queued at the bank's counter: 41 us each on a 40^3 grid's levels, 5 now).
 // The lanes of this lane's run, all of them active.
 __device__ __forceinline__ unsigned long long bank_run(int gb)
 {
@@ -311,9 +321,22 @@ __global__ void k_dp_ent_bank_counts(int n_fine_banks, int bank, const int* row_
     if(b < n_fine_banks) bank_cnt[b] = row_off[(b + 1) * bank] - row_off[b * bank];
 }
 
+// Inclusive prefix sum over a wave by lane moves (all lanes active): four
+// shifts inside the rows of 16, then the rows' last lanes to the rows behind.
+__device__ __forceinline__ int wave_prefix(int v)
+{
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr:1
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);  // row_shr:2
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);  // row_shr:4
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);  // row_shr:8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
+    return v;
+}
+
 // the greedy tile that starts at r0 (build_spmv_layout's cut, from any r0).
 // Bound by the chain of row searches behind one start: a thread that adds its
-// rows one by one makes ~100 dependent ones (165 us on 88,922 rows).  Here a
+// rows one by one makes ~100 dependent ones (165 us on 68,921 rows, 36 now).  Here a
 // wave takes a start, its lanes 64 rows at a time: each lane finds what its row
 // adds, a prefix sum finds the row that no longer fits.  A workgroup takes
 // kSlStarts consecutive starts, whose tiles can only reach the next
@@ -371,13 +394,7 @@ __global__ void __launch_bounds__(kSlThreads) k_dp_sl_next(int n, const int* row
             int q = 0;
             if(r < r_end)
                 q = (s_ptr[r + 1 - R] - s_diag[r - R]) + (first_ge_s(s_ptr[r - R], s_diag[r - R], r0) - s_ptr[r - R]);
-            int sum = q;
-#pragma unroll
-            for(int d = 1; d < 64; d <<= 1)
-            {
-                const int o = __shfl_up(sum, d);
-                if(lane >= d) sum += o;
-            }
+            const int sum = wave_prefix(q);
             const unsigned long long stop = __ballot(r >= r_end || k + sum > cap);
             if(stop)
             {
@@ -399,7 +416,7 @@ __global__ void __launch_bounds__(kSlThreads) k_dp_sl_next(int n, const int* row
 
 // The chain of tiles from row 0, one workgroup, in windows of the tile ends
 // staged in LDS (each step r -> nxt[r] advances by 1..256 rows).  One thread
-// walking the window is a chain of ~300 LDS reads (63 us on 88,922 rows), so
+// walking the window is a chain of ~300 LDS reads (63 us on 68,921 rows, 24 now), so
 // the window is cut into segments: for each of the 256 rows where the chain
 // can enter one, a thread walks it to its end; one thread then links the
 // segments, and a thread per segment writes its tiles.
@@ -493,7 +510,7 @@ __global__ void __launch_bounds__(kThreads) k_dp_sl_tile_counts(int n_tiles, int
 // first column (s_below) and from its diagonal on (s_diag) are kept, so an
 // entry's place follows from its own index.  Columns are searched in LDS when
 // the tile's fit kFillCols (a thread per row walking and searching in global
-// memory: 75 us on 88,922 rows).
+// memory: 75 us on 68,921 rows, 18 now).
 constexpr int kFillCols = 6144;
 
 __global__ void __launch_bounds__(kThreads) k_dp_sl_fill(int n_tiles, int n, const int* ts, const int* kept,
@@ -631,11 +648,17 @@ hipError_t dp_fill(int* p, int value, long long n, hipStream_t st)
 }
 
 hipError_t dp_csr_items(long long nb, const int* rows, const int* cols, DpSystems sys, const int* e2i, int n_rows,
-                        int bits, uint64_t* keys, int* vals, int* row_cnt, int* diag_src, int* err, hipStream_t st)
+                        int bits, uint64_t* keys, int* vals, int* diag_src, int* err, hipStream_t st)
 {
     if(nb <= 0) return hipSuccess;
     hipLaunchKernelGGL(k_dp_csr_items, dim3(grid_for(nb)), dim3(kThreads), 0, st, nb, rows, cols, sys, e2i, n_rows,
-                       bits, keys, vals, row_cnt, diag_src, err);
+                       bits, keys, vals, diag_src, err);
+    return hipGetLastError();
+}
+
+hipError_t dp_row_starts(long long n, const uint64_t* keys, int bits, int n_rows, int* row_ptr, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_dp_row_starts, dim3(grid_for(n + 1)), dim3(kThreads), 0, st, n, keys, bits, n_rows, row_ptr);
     return hipGetLastError();
 }
 
@@ -652,7 +675,7 @@ hipError_t dp_gal_items(int lvl, long long n, const int* rows, const int* cols, 
                         uint64_t* keys, int* vals, int* n_valid, hipStream_t st)
 {
     if(n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_dp_gal_items, dim3(grid_for(n)), dim3(kThreads), 0, st, lvl, n, rows, cols, EI, EJ, ES,
+    hipLaunchKernelGGL(k_dp_gal_items, dim3(grid_for(n, 4 * kThreads)), dim3(kThreads), 0, st, lvl, n, rows, cols, EI, EJ, ES,
                        e_prev, sys, gn_all, lvl_begin, bits, keys, vals, n_valid);
     return hipGetLastError();
 }

@@ -49,11 +49,12 @@ struct DpSystems
 // [0, n_ext_s)) becomes key (R << bits | C) with value k in row R =
 // e2i[ext_off[s] + rows[k]] and, off the diagonal, key (C << bits | R) with
 // value k | bit 31 in row C; a diagonal block's second slot is the sentinel
-// row n_rows.  Counts entries per row (row_cnt, zeroed), records the last
-// diagonal block of each row (diag_src, filled with -1) and flags an index
-// out of range in *err.
+// row n_rows.  Records the last diagonal block of each row (diag_src, filled
+// with -1) and flags an index out of range in *err.
 hipError_t dp_csr_items(long long nb, const int* rows, const int* cols, DpSystems sys, const int* e2i, int n_rows,
-                        int bits, uint64_t* keys, int* vals, int* row_cnt, int* diag_src, int* err, hipStream_t st);
+                        int bits, uint64_t* keys, int* vals, int* diag_src, int* err, hipStream_t st);
+// row_ptr[0 .. n_rows] of the n sorted items (row_ptr[n_rows]: where the sentinels begin)
+hipError_t dp_row_starts(long long n, const uint64_t* keys, int bits, int n_rows, int* row_ptr, hipStream_t st);
 // col / entry_src of the first nnz sorted items
 hipError_t dp_csr_fill(long long nnz, const uint64_t* keys, const int* vals, int bits, int* col, int* entry_src,
                        hipStream_t st);

@@ -117,22 +117,20 @@ void Solver::build_structure_on_device(hipStream_t st)
     d_dp_keys2_.alloc(n_items);
     d_dp_vals_.alloc(n_items);
     d_dp_vals2_.alloc(n_items);
-    d_dp_cnt_.alloc((size_t)n_rows + 1);
     d_diag_src_.alloc(n_rows);
     d_dp_err_.alloc(2);
-    check(dp_fill(d_dp_cnt_.ptr, 0, (long long)n_rows + 1, st), "fill");
     check(dp_fill(d_diag_src_.ptr, -1, n_rows, st), "fill");
     check(dp_fill(d_dp_err_.ptr, 0, 2, st), "fill");
     check(dp_csr_items(nb, d_dp_rows_.ptr, d_dp_cols_.ptr, sys, d_e2i_.ptr, n_rows, bits, d_dp_keys_.ptr,
-                       d_dp_vals_.ptr, d_dp_cnt_.ptr, d_diag_src_.ptr, d_dp_err_.ptr, st),
+                       d_dp_vals_.ptr, d_diag_src_.ptr, d_dp_err_.ptr, st),
           "block CSR items");
-    size_t tmp = std::max(dp_sort_bytes(n_items, 2 * bits), dp_scan_bytes((long long)n_rows + 1));
+    size_t tmp = dp_sort_bytes(n_items, 2 * bits);
     d_dp_tmp_.alloc(tmp);
     check(dp_sort(d_dp_tmp_.ptr, tmp, d_dp_keys_.ptr, d_dp_keys2_.ptr, d_dp_vals_.ptr, d_dp_vals2_.ptr, n_items,
                   2 * bits, st),
           "block CSR sort");
     d_row_ptr_.alloc((size_t)n_rows + 1);
-    check(dp_scan(d_dp_tmp_.ptr, tmp, d_dp_cnt_.ptr, d_row_ptr_.ptr, (long long)n_rows + 1, st), "row scan");
+    check(dp_row_starts(n_items, d_dp_keys2_.ptr, bits, n_rows, d_row_ptr_.ptr, st), "row starts");
     const int* rb = read_ints({d_dp_err_.ptr, d_row_ptr_.ptr + n_rows}, st);
     if(rb[0]) throw std::invalid_argument("block index out of range");
     P.nnz = rb[1];
