@@ -73,13 +73,6 @@ def _busy_median(durations):
     return b[len(b) // 2]
 
 
-def mas_local_variant(waves):
-    """Template arguments after the element type of the FP32 MAS local kernel
-    the variant code runs: 4 / 8 waves, 5 / 9 the same with the inverse
-    staged through LDS."""
-    return {4: "4, false", 8: "8, false", 5: "4, true", 9: "8, true"}[waves]
-
-
 def compare(bench_json, trace_csv):
     """bench.py's per-kernel event times (the 64-system batch's FP32 kernels,
     or the 40^3 workload's for --fem40-only) beside the trace's busy medians."""
@@ -92,9 +85,8 @@ def compare(bench_json, trace_csv):
         obj = bench["fem40c"]
         us = {k: v["us"] for k, v in obj["roofline"]["per_kernel"].items()}
     tiling = obj["spmv_tiling"]["entries_per_thread"]
-    waves = obj["spmv_tiling"].get("mas_local", {}).get("fp32", {}).get("waves", 4)
     nt = "true" if obj["spmv_tiling"].get("nontemporal") else "false"
-    names = {"spmv": f"k_spmv_fused<{tiling}, {nt},", "mas_local": f"k_mas_local<32, float, {mas_local_variant(waves)}>",
+    names = {"spmv": f"k_spmv_fused<{tiling}, {nt},", "mas_local": "k_mas_lanes<32, float,",
              "precond_finish": "k_precond_finish", "update": "k_update"}
     d = collections.defaultdict(list)
     for r in csv.DictReader(open(trace_csv)):

@@ -95,16 +95,13 @@ def algorithmic_bytes(info, n_vertices, prec_bytes):
     }
 
 
-KERNEL_PREFIX = {"spmv": "k_spmv_fused", "mas_local": "k_mas_local<32, float,", "update": "k_update",
+KERNEL_PREFIX = {"spmv": "k_spmv_fused", "mas_local": "k_mas_lanes<32, float,", "update": "k_update",
                  "precond_finish": "k_precond_finish"}
 
 
-def measured_traffic(kernel, workload_is_default, spmv_entries, summary="fem40c_hbm_traffic.json", waves=None,
-                     spmv_nt=False):
+def measured_traffic(kernel, workload_is_default, spmv_entries, summary="fem40c_hbm_traffic.json", spmv_nt=False):
     """HBM bytes per launch of `kernel` (the SpMV at `spmv_entries` per
-    thread with nontemporal matrix loads or not, the FP32 MAS local kernel at
-    `waves` waves per workgroup) from the
-    committed counter summary of this workload (FETCH_SIZE + WRITE_SIZE runs,
+    thread with nontemporal matrix loads or not) from the committed counter summary of this workload (FETCH_SIZE + WRITE_SIZE runs,
     copy-calibrated), or None."""
     path = os.path.join(ROOT, "profiles", summary)
     if not workload_is_default or not os.path.exists(path):
@@ -112,9 +109,6 @@ def measured_traffic(kernel, workload_is_default, spmv_entries, summary="fem40c_
     data = json.load(open(path))["kernels"]
     want = (f"k_spmv_fused<{spmv_entries}, {'true' if spmv_nt else 'false'}," if kernel == "spmv"
             else KERNEL_PREFIX[kernel])
-    if kernel == "mas_local" and waves:
-        from agipc_learning_amd.prof_summary import mas_local_variant
-        want = f"{KERNEL_PREFIX[kernel]} {mas_local_variant(waves)}>"
     for name, v in data.items():
         if name.startswith(want):
             return int(v["bytes"])
@@ -357,10 +351,10 @@ def batch_leg(args):
     sols = {}
     tiling["mas_local"] = {}
     for prec in precs:
-        # the MAS local variant for this precision (VALU waves per workgroup, or MFMA)
+        # the automatic MAS local kernel: in every precision the fastest, here and on the 40^3 grid
         s.build(prec)
-        tiling["mas_local"][prec] = s.autotune_mas(20)
-        log(f"step: batch64 {prec} ({args.warmup} warmup + {args.steps} steps), local variant "
+        tiling["mas_local"][prec] = dict(waves=0, ms=s.time_kernel(0, 20))
+        log(f"step: batch64 {prec} ({args.warmup} warmup + {args.steps} steps), local solve "
             f"{tiling['mas_local'][prec]}")
         for i in range(args.warmup):
             step(prec, i + 1)
@@ -404,9 +398,7 @@ def batch_leg(args):
             out["roofline"] = {"bound": "hbm", "kernel": dom, "achieved": round(ach, 1), "peak": HBM_PEAK_GBS,
                                "unit": "GB/s", "frac": round(ach / HBM_PEAK_GBS, 4),
                                "traffic": measured_traffic(dom, True, tiling["entries_per_thread"],
-                                                           "batch64_hbm_traffic.json",
-                                                           tiling["mas_local"]["fp32"]["waves"],
-                                                           tiling["nontemporal"]),
+                                                           "batch64_hbm_traffic.json", tiling["nontemporal"]),
                                "algorithmic_bytes": alg[dom], "avg_us": kern[dom],
                                "per_kernel": {k: {"us": kern[k], "GB/s": out[prec]["kernels_GBs"][k],
                                                   "algorithmic_bytes": alg[k]} for k in kern}}
@@ -674,8 +666,8 @@ def fem40_leg(args, structure=True):
     tiling["mas_local"] = {}
     for prec in precs:
         s.build(prec)
-        tiling["mas_local"][prec] = s.autotune_mas(50)
-        log(f"step: fem40c {prec} ({args.warmup} warmup + {args.fem40_steps} steps), local variant "
+        tiling["mas_local"][prec] = dict(waves=0, ms=s.time_kernel(0, 50))
+        log(f"step: fem40c {prec} ({args.warmup} warmup + {args.fem40_steps} steps), local solve "
             f"{tiling['mas_local'][prec]}")
         ms, st = run(prec, args.fem40_steps, args.warmup)
         if st["failure"] != 0 or st["rel_res_true"] > args.tol * (1 + 1e-6):
@@ -709,7 +701,6 @@ def fem40_leg(args, structure=True):
                 "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
                 "traffic": measured_traffic(dominant, (args.n, args.contacts, args.levels) == (40, 20000, 4),
                                             tiling["entries_per_thread"],
-                                            waves=tiling["mas_local"]["fp32"]["waves"],
                                             spmv_nt=tiling["nontemporal"]),
                 "algorithmic_bytes": alg[dominant], "avg_us": round(kern[dominant], 2),
                 "per_kernel": {k: {"us": round(kern[k], 2), "GB/s": round(alg[k] / (kern[k] * 1e-6) / 1e9, 1)}
