@@ -9,6 +9,7 @@
 
 #include "device.hpp"
 #include "spmv_layout.hpp"
+#include "wave_prefix.hpp"
 
 namespace masx
 {
@@ -319,19 +320,6 @@ __global__ void k_dp_ent_bank_counts(int n_fine_banks, int bank, const int* row_
 {
     const int b = blockIdx.x * blockDim.x + threadIdx.x;
     if(b < n_fine_banks) bank_cnt[b] = row_off[(b + 1) * bank] - row_off[b * bank];
-}
-
-// Inclusive prefix sum over a wave by lane moves (all lanes active): four
-// shifts inside the rows of 16, then the rows' last lanes to the rows behind.
-__device__ __forceinline__ int wave_prefix(int v)
-{
-    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr:1
-    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);  // row_shr:2
-    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);  // row_shr:4
-    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);  // row_shr:8
-    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
-    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
-    return v;
 }
 
 // the greedy tile that starts at r0 (build_spmv_layout's cut, from any r0).

@@ -93,29 +93,36 @@ __global__ void __launch_bounds__(256) k_h_init(Lv lv, int n_slots, long long ma
 }
 
 // Input checks, the level-0 adjacency (own bit for slots holding a vertex) and
-// the starting node of every vertex.
+// the starting node of every vertex.  Eight lanes share a vertex's neighbours
+// and read a neighbour's list four words at a time: a thread per vertex, word
+// by word, was a chain of ~100 reads (68,921 vertices: 23 us, 17.5 now).
+constexpr int kCheckLanes = 8;
 __global__ void __launch_bounds__(256) k_h_validate(Lv lv, int n_fem, int n_slots, int bank, const uint32_t* start,
                                                     const uint32_t* num, const uint32_t* list, long long list_len,
                                                     const int* p2r, const int* r2p, int* id, uint32_t* adj)
 {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    const long long at = blockIdx.x * (long long)blockDim.x + threadIdx.x;
     int flag = 0;
-    if(t < n_slots)
+    if(at < n_slots)
     {
-        const int r = p2r[t];
+        const int t = (int)at, r = p2r[t];
         if(r < -1 || r >= n_fem || (r >= 0 && r2p[r] != t)) flag |= kBadPartition;
         adj[t] = r >= 0 ? (1u << (t % bank)) : 0u;
     }
-    if(t < n_fem)
+    if(at < (long long)n_fem * kCheckLanes)
     {
-        const int s = r2p[t];
-        if(s < 0 || s >= n_slots || p2r[s] != t) flag |= kBadPartition;
-        id[t] = s >= 0 && s < n_slots ? s : 0;
+        const int t = (int)(at / kCheckLanes), lane = (int)(at % kCheckLanes);
+        if(lane == 0)
+        {
+            const int s = r2p[t];
+            if(s < 0 || s >= n_slots || p2r[s] != t) flag |= kBadPartition;
+            id[t] = s >= 0 && s < n_slots ? s : 0;
+        }
         const unsigned long long b = start[t], c = num[t];
         if(b + c > (unsigned long long)list_len)
             flag |= kBadList;
         else
-            for(unsigned long long i = 0; i < c; ++i)
+            for(unsigned long long i = lane; i < c; i += kCheckLanes)
             {
                 const uint32_t u = list[b + i];
                 if(u >= (uint32_t)n_fem)
@@ -123,11 +130,16 @@ __global__ void __launch_bounds__(256) k_h_validate(Lv lv, int n_fem, int n_slot
                     flag |= kBadNeighbor;
                     continue;
                 }
-                // t must appear in u's list (u's own range is checked by u's thread)
+                // t must appear in u's list (u's own range is checked by u's lanes)
                 const unsigned long long bu = start[u], cu = num[u];
                 if(bu + cu > (unsigned long long)list_len) continue;
                 bool back = false;
-                for(unsigned long long k = 0; k < cu && !back; ++k) back = list[bu + k] == (uint32_t)t;
+                for(unsigned long long k = 0; k < cu && !back; k += 4)
+                {
+#pragma unroll
+                    for(int q = 0; q < 4; ++q)
+                        back |= list[bu + (k + q < cu ? k + q : k)] == (uint32_t)t;
+                }
                 if(!back) flag |= kAsymmetric;
             }
     }
@@ -477,8 +489,8 @@ void DeviceHierarchy::build(int n_fem, int n_slots, int bank, int levels, const 
     const int per = 64 / bank;
     hipLaunchKernelGGL(k_h_init, dim3(blocks((long long)max_slots, 256)), dim3(256), 0, st, lv, n_slots,
                        (long long)max_slots, (long long)max_banks, going_next_, ncomp_all_);
-    hipLaunchKernelGGL(k_h_validate, dim3(blocks(std::max(n_fem, n_slots), 256)), dim3(256), 0, st, lv, n_fem,
-                       n_slots, bank, start, num, list, list_len, p2r, r2p, id_, adj_);
+    hipLaunchKernelGGL(k_h_validate, dim3(blocks(std::max((long long)n_fem * kCheckLanes, (long long)n_slots), 256)),
+                       dim3(256), 0, st, lv, n_fem, n_slots, bank, start, num, list, list_len, p2r, r2p, id_, adj_);
     // grids are sized by the bound n_slots; kernels read the level sizes
     for(int level = 0; level < L; ++level)
     {

@@ -211,3 +211,14 @@ def test_device_structure_around_tile_ends(sizes, per_row, hub):
             s.set_spmv_tiling(entries)
         for name in native.Solver.PLAN_ARRAYS:
             assert np.array_equal(want.plan_array(name), got.plan_array(name)), (entries, name)
+
+
+@pytest.mark.parametrize("n", [1, 63, 65, 511, 513, 2047, 2049, 131072, 140000])
+def test_device_morton_around_rounds_and_chunks(n):
+    """The device partition equals the host's where waves, tiles and the scan's
+    kept counts (64 tiles) end, with many equal codes (their order is the index order)."""
+    rng = np.random.default_rng(n)
+    pos = rng.integers(0, 9, (n, 3)).astype(np.float64)
+    p2r, r2p = native.DeviceMorton().partition(dev(pos))
+    want_p2r, want_r2p = native.morton_partition(pos)
+    assert np.array_equal(host(p2r), want_p2r) and np.array_equal(host(r2p), want_r2p)
