@@ -2970,7 +2970,7 @@ __global__ void __launch_bounds__(256) k_rows_from_ext64(const int* __restrict__
 // more than a chunk takes several chunks.  Bound by the blocks' bytes, each
 // read for its row and, transposed, for its column (the second mostly from
 // the caches: rows run in Morton order and each XCD has a contiguous run).
-// 226,981 rows, 1.77 M upper blocks: one thread per row 134 us.
+// 226,981 rows, 1.77 M upper blocks: one thread per row 134 us, the whole product 166; now 70.
 constexpr int kRows64 = 64, kEntries64 = 85 * 12;
 __global__ void __launch_bounds__(256) k_spmv64(DevData d, const int* __restrict__ int_to_ext,
                                                 const double* __restrict__ x, double a, double b,
