@@ -3048,9 +3048,10 @@ __global__ void __launch_bounds__(256) k_gather_blocks(const double* src, const 
 
 // *differs (host-visible, zero before) := 1 unless block k of the selection has
 // row rows[idx[k]] - offset == want_rows[k], column likewise (idx null: k), and
-// the pairs equal want_pairs.
+// the pairs equal want_pairs.  An index from n_all on differs without a read.
 __global__ void __launch_bounds__(256) k_structure_differs(const int* __restrict__ rows, const int* __restrict__ cols,
-                                                           const uint32_t* __restrict__ idx, int offset, int n,
+                                                           const uint32_t* __restrict__ idx, long long n_all,
+                                                           int offset, int n,
                                                            const int* __restrict__ want_rows,
                                                            const int* __restrict__ want_cols,
                                                            const int* __restrict__ pairs,
@@ -3062,7 +3063,7 @@ __global__ void __launch_bounds__(256) k_structure_differs(const int* __restrict
     if(t < n)
     {
         const uint32_t k = idx ? idx[t] : (uint32_t)t;
-        bad = rows[k] - offset != want_rows[t] || cols[k] - offset != want_cols[t];
+        bad = k >= n_all || rows[k] - offset != want_rows[t] || cols[k] - offset != want_cols[t];
     }
     if(t < n_pair_ints) bad |= pairs[t] != want_pairs[t];
     if(bad) *(volatile int*)differs = 1;
@@ -3436,14 +3437,14 @@ hipError_t launch_spmv64(const DevData& d, const int* i2e, const double* x, doub
     return hipSuccess;
 }
 
-hipError_t launch_structure_differs(const int* rows, const int* cols, const uint32_t* idx, int offset, int n,
-                                    const int* want_rows, const int* want_cols, const int* pairs,
+hipError_t launch_structure_differs(const int* rows, const int* cols, const uint32_t* idx, long long n_all,
+                                    int offset, int n, const int* want_rows, const int* want_cols, const int* pairs,
                                     const int* want_pairs, int n_pair_ints, int* differs, hipStream_t st)
 {
     const int m = std::max(n, n_pair_ints);
     if(m <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_structure_differs, dim3(blocks_for(m, 256)), dim3(256), 0, st, rows, cols, idx, offset, n,
-                       want_rows, want_cols, pairs, want_pairs, n_pair_ints, differs);
+    hipLaunchKernelGGL(k_structure_differs, dim3(blocks_for(m, 256)), dim3(256), 0, st, rows, cols, idx, n_all,
+                       offset, n, want_rows, want_cols, pairs, want_pairs, n_pair_ints, differs);
     MASX_CHECK_LAUNCH();
     return hipSuccess;
 }

@@ -58,9 +58,9 @@ hipError_t launch_true_residual(const DevData& d, int n_wg, int report_only, hip
 hipError_t launch_rows_from_ext64(const int* i2e, const double* src, double* dst, int n_rows, hipStream_t st);
 hipError_t launch_spmv64(const DevData& d, const int* i2e, const double* x, double a, double b, double* y,
                          hipStream_t st);
-// sets *differs (host-visible) unless the selected structure and the pairs are the wanted ones
-hipError_t launch_structure_differs(const int* rows, const int* cols, const uint32_t* idx, int offset, int n,
-                                    const int* want_rows, const int* want_cols, const int* pairs,
+// sets *differs (host-visible) unless the selected structure (every index below n_all) and the pairs are the wanted ones
+hipError_t launch_structure_differs(const int* rows, const int* cols, const uint32_t* idx, long long n_all,
+                                    int offset, int n, const int* want_rows, const int* want_cols, const int* pairs,
                                     const int* want_pairs, int n_pair_ints, int* differs, hipStream_t st);
 hipError_t launch_gather_blocks(const double* src, const uint32_t* idx, double* dst, long long n, hipStream_t st);
 

@@ -77,6 +77,20 @@ void hip_ok(hipError_t e)
 {
     if(e != hipSuccess) throw std::runtime_error(std::string("HIP: ") + hipGetErrorString(e));
 }
+
+// Whole items of `bytes` from p to the end of the allocation it lies in; -1
+// where HIP knows no allocation there.
+long long room(const void* p, size_t bytes)
+{
+    hipDeviceptr_t base = nullptr;
+    size_t         size = 0;
+    if(hipMemGetAddressRange(&base, &size, const_cast<void*>(p)) != hipSuccess)
+    {
+        (void)hipGetLastError();
+        return -1;
+    }
+    return (long long)((size - (size_t)((const char*)p - (const char*)base)) / bytes);
+}
 }  // namespace
 
 struct masx_mas
@@ -774,17 +788,27 @@ int masx_mas_set_preconditioner_bcoo(masx_mas* m, const double* d_values, const 
         require(cp_num == 0 || d_pairs != nullptr, "null contact pairs");
         hipStream_t st = as_stream(stream);
         const int   n_pair_ints = 4 * cp_num;
+        // the kernels below read the caller's arrays by the caller's counts and
+        // indices: none may lead past an allocation
+        const long long idx_room = d_indices ? room(d_indices, sizeof(uint32_t)) : triplet_num;
+        const long long pair_room = n_pair_ints ? room(d_pairs, sizeof(int)) : 0;
+        require(idx_room < 0 || idx_room >= triplet_num, "fewer indices than selected blocks");
+        require(pair_room < 0 || pair_room >= n_pair_ints, "fewer contact pairs than their count");
+        const long long n_all_max = std::min(
+            {room(d_values, 9 * sizeof(double)), room(d_rows, sizeof(int)), room(d_cols, sizeof(int))});
         // the structure of the call before, compared on the device: a Newton
         // step that keeps it costs one flag instead of its download
-        bool same = m->solver && triplet_num == m->n_blocks && n_pair_ints == m->n_pair_ints;
+        bool same = m->solver && triplet_num == m->n_blocks && n_pair_ints == m->n_pair_ints && n_all_max >= 0
+                    && idx_room >= 0 && pair_room >= 0;
         if(same)
         {
             if(!m->h_differs) hip_ok(hipHostMalloc((void**)&m->h_differs, 64, hipHostMallocCoherent | hipHostMallocMapped));
             int* d_differs = nullptr;
             hip_ok(hipHostGetDevicePointer((void**)&d_differs, m->h_differs, 0));
             *(volatile int*)m->h_differs = 0;
-            hip_ok(masx::launch_structure_differs(d_rows, d_cols, d_indices, offset, triplet_num, m->d_rows.ptr,
-                                                  m->d_cols.ptr, d_pairs, m->d_pairs.ptr, n_pair_ints, d_differs, st));
+            hip_ok(masx::launch_structure_differs(d_rows, d_cols, d_indices, n_all_max, offset, triplet_num,
+                                                  m->d_rows.ptr, m->d_cols.ptr, d_pairs, m->d_pairs.ptr, n_pair_ints,
+                                                  d_differs, st));
             if(hipStreamSynchronize(st) != hipSuccess) throw std::runtime_error("stream sync failed");
             same = *(volatile int*)m->h_differs == 0;
         }
@@ -806,6 +830,7 @@ int masx_mas_set_preconditioner_bcoo(masx_mas* m, const double* d_values, const 
             uint32_t max_idx = 0;
             for(uint32_t v : idx) max_idx = std::max(max_idx, v);
             const size_t n_all = triplet_num ? (size_t)max_idx + 1 : 0;
+            require(n_all_max < 0 || (long long)n_all <= n_all_max, "selected block outside the matrix");
             std::vector<int> all_r(n_all), all_c(n_all);
             if(n_all)
             {

@@ -142,6 +142,19 @@ def test_lane_tiles_agree_with_the_block_diagonal_layout(bank, precision, n, con
         assert st["failure"] == 0 and st["rel_res_true"] <= 1e-4 * (1 + 1e-6)
 
 
+def mas_object(w, m=None, levels=0):
+    """A preconditioner object of the mesh of w (or m given that mesh)."""
+    from agipc_learning_amd import workloads as W
+
+    p2r, r2p = native.morton_partition(w["positions"])
+    start, num, lst = W.neighbors(w["n_vertices"], w["tets"])
+    m = native.MasPreconditioner(32) if m is None else m
+    m.init_neighbor(w["n_vertices"], 0, len(lst), len(p2r))
+    m.upload(lst, start, num, p2r, r2p)
+    m.init_matrix(levels)
+    return m
+
+
 def test_mas_object_sees_a_structure_of_the_same_size():
     """A call with as many blocks and pairs as the last but another order of
     blocks, or other pairs, is not taken for the same structure: its apply
@@ -150,17 +163,11 @@ def test_mas_object_sees_a_structure_of_the_same_size():
 
     w = W.fem_grid(9, n_contacts=120, seed=4, young_sigma=0.5)
     nv, nb = w["n_vertices"], len(w["rows"])
-    p2r, r2p = native.morton_partition(w["positions"])
-    start, num, lst = W.neighbors(nv, w["tets"])
     rng = np.random.default_rng(8)
     R = dev(rng.standard_normal(3 * nv))
 
     def fresh():
-        m = native.MasPreconditioner(32)
-        m.init_neighbor(nv, 0, len(lst), len(p2r))
-        m.upload(lst, start, num, p2r, r2p)
-        m.init_matrix()
-        return m
+        return mas_object(w)
 
     def apply(m, order, pairs, select=True):
         idx = dev(order.astype(np.int32)) if select else None
@@ -183,6 +190,38 @@ def test_mas_object_sees_a_structure_of_the_same_size():
     with pytest.raises(RuntimeError):
         m.set_preconditioner_bcoo(dev(w["vals"]), dev(w["rows"]), dev(w["cols"]), dev(plain.astype(np.int32)), 1, nb,
                                   pairs=dev(np.asarray(w["pairs"], np.int32)), cp_num=len(w["pairs"]))
+
+
+def test_mas_object_refuses_a_selection_outside_the_matrix():
+    """After an accepted call, a call of the same counts whose indices, or whose
+    count of indices or pairs, lead past the caller's arrays is refused on the
+    host before anything reads there, and leaves the object as it was."""
+    from agipc_learning_amd import workloads as W
+
+    w = W.fem_grid(9, n_contacts=120, seed=4, young_sigma=0.5)
+    nv, nb = w["n_vertices"], len(w["rows"])
+    vals, rows, cols, idx = dev(w["vals"]), dev(w["rows"]), dev(w["cols"]), dev(np.arange(nb, dtype=np.int32))
+    # more pairs than a small tensor's allocation (2 MiB at most) can hold
+    many = dev(np.tile(np.asarray(w["pairs"], np.int32).reshape(-1, 4), (1700, 1)))
+    R = dev(np.random.default_rng(8).standard_normal(3 * nv))
+    m = mas_object(w)
+    m.set_preconditioner_bcoo(vals, rows, cols, idx, 0, nb, pairs=many, cp_num=len(many))
+    want = torch.zeros_like(R)
+    m.preconditioning(R, want)
+    far = idx.clone()
+    far[nb // 2] = 1 << 27
+    with pytest.raises(RuntimeError, match="outside the matrix"):
+        m.set_preconditioner_bcoo(vals, rows, cols, far, 0, nb, pairs=many, cp_num=len(many))
+    with pytest.raises(RuntimeError, match="fewer contact pairs"):
+        m.set_preconditioner_bcoo(vals, rows, cols, idx, 0, nb, pairs=many[:4].clone(), cp_num=len(many))
+    with pytest.raises(RuntimeError, match="fewer indices"):
+        m.set_preconditioner_bcoo(vals, rows, cols, idx, 0, 1 << 27, pairs=many, cp_num=len(many))
+    got = torch.zeros_like(R)
+    m.preconditioning(R, got)
+    assert np.array_equal(host(got), host(want))
+    m.set_preconditioner_bcoo(vals, rows, cols, idx, 0, nb, pairs=many, cp_num=len(many))
+    m.preconditioning(R, got)
+    assert np.array_equal(host(got), host(want))
 
 
 @pytest.mark.parametrize("sizes,per_row,hub", [((1,), 0, 0), ((256, 257), 0, 0), ((33100, 40), 0, 0), ((129, 127), 2, 90),
