@@ -3055,10 +3055,10 @@ __global__ void __launch_bounds__(256) k_structure_differs(const int* __restrict
                                                            const int* __restrict__ want_rows,
                                                            const int* __restrict__ want_cols,
                                                            const int* __restrict__ pairs,
-                                                           const int* __restrict__ want_pairs, int n_pair_ints,
+                                                           const int* __restrict__ want_pairs, long long n_pair_ints,
                                                            int* differs)
 {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    const long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x;
     bool bad = false;
     if(t < n)
     {
@@ -3439,9 +3439,9 @@ hipError_t launch_spmv64(const DevData& d, const int* i2e, const double* x, doub
 
 hipError_t launch_structure_differs(const int* rows, const int* cols, const uint32_t* idx, long long n_all,
                                     int offset, int n, const int* want_rows, const int* want_cols, const int* pairs,
-                                    const int* want_pairs, int n_pair_ints, int* differs, hipStream_t st)
+                                    const int* want_pairs, long long n_pair_ints, int* differs, hipStream_t st)
 {
-    const int m = std::max(n, n_pair_ints);
+    const long long m = std::max((long long)n, n_pair_ints);
     if(m <= 0) return hipSuccess;
     hipLaunchKernelGGL(k_structure_differs, dim3(blocks_for(m, 256)), dim3(256), 0, st, rows, cols, idx, n_all,
                        offset, n, want_rows, want_cols, pairs, want_pairs, n_pair_ints, differs);

@@ -61,7 +61,7 @@ hipError_t launch_spmv64(const DevData& d, const int* i2e, const double* x, doub
 // sets *differs (host-visible) unless the selected structure (every index below n_all) and the pairs are the wanted ones
 hipError_t launch_structure_differs(const int* rows, const int* cols, const uint32_t* idx, long long n_all,
                                     int offset, int n, const int* want_rows, const int* want_cols, const int* pairs,
-                                    const int* want_pairs, int n_pair_ints, int* differs, hipStream_t st);
+                                    const int* want_pairs, long long n_pair_ints, int* differs, hipStream_t st);
 hipError_t launch_gather_blocks(const double* src, const uint32_t* idx, double* dst, long long n, hipStream_t st);
 
 // Device arrays of doubles copied into one array by one launch: segment s,

@@ -102,7 +102,8 @@ struct masx_mas
     bool uploaded = false, matrix_ready = false;
     // structure of the last set_preconditioner_bcoo call: block count, pair
     // ints, and on the device its rows and columns (offset subtracted) and pairs
-    int n_blocks = -1, n_pair_ints = 0;
+    int       n_blocks    = -1;
+    long long n_pair_ints = 0;
     masx::DeviceArray<int> d_rows, d_cols, d_pairs;
     std::unique_ptr<masx_solver> solver;
     int* h_differs = nullptr;  // coherent pinned: the structure comparison's answer
@@ -787,7 +788,7 @@ int masx_mas_set_preconditioner_bcoo(masx_mas* m, const double* d_values, const 
         require(cp_num >= 0, "negative pair count");
         require(cp_num == 0 || d_pairs != nullptr, "null contact pairs");
         hipStream_t st = as_stream(stream);
-        const int   n_pair_ints = 4 * cp_num;
+        const long long n_pair_ints = 4 * (long long)cp_num;
         // the kernels below read the caller's arrays by the caller's counts and
         // indices: none may lead past an allocation
         const long long idx_room = d_indices ? room(d_indices, sizeof(uint32_t)) : triplet_num;

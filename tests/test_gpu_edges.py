@@ -224,6 +224,20 @@ def test_mas_object_refuses_a_selection_outside_the_matrix():
     assert np.array_equal(host(got), host(want))
 
 
+@pytest.mark.parametrize("cp_num", [1 << 29, 1 << 30, 2**31 - 1])
+def test_mas_object_counts_pairs_in_64_bits(cp_num):
+    """Pair counts whose four indices a pair pass 2^31 are refused for an array
+    that cannot hold them (in 32 bits 2^30 pairs count as none)."""
+    from agipc_learning_amd import workloads as W
+
+    w = W.fem_grid(4, n_contacts=10, seed=4, young_sigma=0.5)
+    nb = len(w["rows"])
+    m = mas_object(w)
+    with pytest.raises(RuntimeError, match="fewer contact pairs"):
+        m.set_preconditioner_bcoo(dev(w["vals"]), dev(w["rows"]), dev(w["cols"]), dev(np.arange(nb, dtype=np.int32)),
+                                  0, nb, pairs=dev(np.asarray(w["pairs"], np.int32)), cp_num=cp_num)
+
+
 @pytest.mark.parametrize("sizes,per_row,hub", [((1,), 0, 0), ((256, 257), 0, 0), ((33100, 40), 0, 0), ((129, 127), 2, 90),
                                                ((700,), 24, 600), ((35000,), 2, 300)])
 def test_device_structure_around_tile_ends(sizes, per_row, hub):
