@@ -107,6 +107,12 @@ struct masx_mas
     masx::DeviceArray<int> d_rows, d_cols, d_pairs;
     std::unique_ptr<masx_solver> solver;
     int* h_differs = nullptr;  // coherent pinned: the structure comparison's answer
+    // the mesh or the hierarchy's levels changed: nothing of the solver holds any more
+    void drop_solver()
+    {
+        solver.reset();
+        n_blocks = -1;
+    }
     ~masx_mas()
     {
         if(h_differs) (void)hipHostFree(h_differs);
@@ -746,6 +752,10 @@ int masx_mas_init_neighbor(masx_mas* m, int vert_num, int collision_node_offset,
     return guard([&] {
         require(m && vert_num >= 1 && total_neighbor_num >= 0, "bad argument");
         require(part_map_size >= vert_num && part_map_size % m->bank == 0, "bad partition size");
+        const bool sizes = vert_num != m->vert_num || total_neighbor_num != m->neighbor_total ||
+                           part_map_size != m->part_map_size;
+        if(sizes || collision_node_offset != m->node_offset) m->drop_solver();
+        if(sizes) m->uploaded = m->matrix_ready = false;  // the arrays held are of the other sizes
         m->vert_num       = vert_num;
         m->node_offset    = collision_node_offset;
         m->neighbor_total = total_neighbor_num;
@@ -760,11 +770,16 @@ int masx_mas_upload(masx_mas* m, const uint32_t* neighbor_list, const uint32_t* 
         require(m && m->vert_num > 0, "init_neighbor must come first");
         require(neighbor_start && neighbor_num && part_to_real && real_to_part, "null argument");
         require(m->neighbor_total == 0 || neighbor_list, "null neighbor list");
-        m->nbr_list.assign(neighbor_list, neighbor_list + m->neighbor_total);
-        m->nbr_start.assign(neighbor_start, neighbor_start + m->vert_num);
-        m->nbr_num.assign(neighbor_num, neighbor_num + m->vert_num);
-        m->part_to_real.assign(part_to_real, part_to_real + m->part_map_size);
-        m->real_to_part.assign(real_to_part, real_to_part + m->vert_num);
+        auto keep = [m](auto& held, const auto* from, int n) {  // the same mesh again keeps its solver
+            if((int)held.size() == n && std::equal(held.begin(), held.end(), from)) return;
+            m->drop_solver();
+            held.assign(from, from + n);
+        };
+        keep(m->nbr_list, neighbor_list, m->neighbor_total);
+        keep(m->nbr_start, neighbor_start, m->vert_num);
+        keep(m->nbr_num, neighbor_num, m->vert_num);
+        keep(m->part_to_real, part_to_real, m->part_map_size);
+        keep(m->real_to_part, real_to_part, m->vert_num);
         m->uploaded = true;
     });
 }
@@ -773,6 +788,7 @@ int masx_mas_init_matrix(masx_mas* m, int levels)
 {
     return guard([&] {
         require(m && m->uploaded, "upload must come first");
+        if(levels != m->levels) m->drop_solver();
         m->levels       = levels;
         m->matrix_ready = true;
     });

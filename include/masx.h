@@ -442,7 +442,8 @@ int masx_mas_set_preconditioner_bcoo(masx_mas* m, const double* d_values, const 
                                      int cp_num, int precision, void* stream);
 /* preconditioning(R, Z) (:2684-2725): device double3 arrays of the FEM range. */
 int masx_mas_preconditioning(masx_mas* m, const double* d_R, double* d_Z, void* stream);
-/* the solver the MAS object drives (introspection) */
+/* the solver the MAS object drives (introspection); another mesh, partition or
+ * level count given to the three calls above frees it */
 masx_solver* masx_mas_solver(masx_mas* m);
 
 #ifdef __cplusplus

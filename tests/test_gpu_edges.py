@@ -238,6 +238,46 @@ def test_mas_object_counts_pairs_in_64_bits(cp_num):
                                   0, nb, pairs=dev(np.asarray(w["pairs"], np.int32)), cp_num=cp_num)
 
 
+def test_mas_object_takes_another_mesh():
+    """One object given another partition, another level count, a smaller and
+    a larger mesh applies as a fresh object does, bit for bit, and asks for the
+    matrix before it applies anything; the same mesh again keeps its solver."""
+    from agipc_learning_amd import workloads as W
+
+    def matrix(m, w):
+        nb = len(w["rows"])
+        m.set_preconditioner_bcoo(dev(w["vals"]), dev(w["rows"]), dev(w["cols"]), dev(np.arange(nb, dtype=np.int32)),
+                                  0, nb)
+
+    def applied(m, w):
+        R = dev(np.random.default_rng(3).standard_normal(3 * w["n_vertices"]))
+        Z = torch.zeros_like(R)
+        m.preconditioning(R, Z)
+        return host(Z)
+
+    w = W.fem_grid(9, seed=4, young_sigma=0.5)
+    turned = dict(w, positions=np.ascontiguousarray(w["positions"][:, ::-1]) * [1.0, -2.0, 0.5])
+    m = None
+    for mesh, levels in ((w, 0), (turned, 0), (turned, 2), (W.fem_grid(5, seed=4), 0), (w, 0)):
+        m = mas_object(mesh, m, levels)
+        with pytest.raises(RuntimeError, match="set_preconditioner_bcoo must come first"):
+            applied(m, mesh)
+        matrix(m, mesh)
+        fresh = mas_object(mesh, None, levels)
+        matrix(fresh, mesh)
+        got, want = applied(m, mesh), applied(fresh, mesh)
+        assert np.array_equal(got, want)
+        kept = m.L.masx_mas_solver(m.h)
+        mas_object(mesh, m, levels)
+        assert m.L.masx_mas_solver(m.h) == kept and np.array_equal(applied(m, mesh), want)
+    small = W.fem_grid(5, seed=4)
+    m.init_neighbor(small["n_vertices"], 0, 0, (small["n_vertices"] + 31) // 32 * 32)
+    with pytest.raises(RuntimeError, match="upload must come first"):  # the arrays held are the other mesh's
+        m.init_matrix()
+    with pytest.raises(RuntimeError, match="init_matrix must come first"):
+        matrix(m, small)
+
+
 @pytest.mark.parametrize("sizes,per_row,hub", [((1,), 0, 0), ((256, 257), 0, 0), ((33100, 40), 0, 0), ((129, 127), 2, 90),
                                                ((700,), 24, 600), ((35000,), 2, 300)])
 def test_device_structure_around_tile_ends(sizes, per_row, hub):
