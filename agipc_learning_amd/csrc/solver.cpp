@@ -844,6 +844,7 @@ void Solver::build(int precision, hipStream_t user)
     const bool prec_changed = precision != precision_;
     precision_ = precision;
     dd_.mas_waves    = effective_mas_waves();  // the factor writes the layout the local kernel reads
+    minv_waves_      = dd_.mas_waves;
     dd_.factor_waves = effective_factor_waves();
     const char* old_minv = d_minv_.ptr;
     d_minv_.alloc(std::max<size_t>(inverse_bytes(), 16));  // reuses the buffer when it fits
@@ -1093,10 +1094,10 @@ void Solver::download_inverse(std::vector<float>& out)
     // words per bank as the local kernels index them: FP32 9 per block, the
     // half block-diagonal layout 5 per block, the MFMA tiles kTileBankHalves / 2,
     // the lane tiles 64 lanes' words
-    const bool f32 = precision_ == kPrecFp32, lanes = dd_.mas_waves == 2;
+    const bool f32 = precision_ == kPrecFp32, lanes = minv_waves_ == 2;
     const size_t stride_words = lanes ? (size_t)64 * lane_tile_words(B, f32)
                                 : precision_ == kPrecFp32 ? nblk * 9
-                                : (B == 32 && dd_.mas_waves == 1) ? (size_t)kTileBankHalves / 2
+                                : (B == 32 && minv_waves_ == 1) ? (size_t)kTileBankHalves / 2
                                                                    : nblk * 5;
     std::vector<uint32_t> raw((size_t)plan_.n_banks * bank_bytes / 4);
     if(!raw.empty()) MASX_HIP(hipMemcpy(raw.data(), d_minv_.ptr, raw.size() * 4, hipMemcpyDeviceToHost));
@@ -1141,7 +1142,7 @@ void Solver::download_inverse(std::vector<float>& out)
                     {
                         std::memcpy(&v, &bw[9 * off + c * len + I], 4);
                     }
-                    else if(B == 32 && dd_.mas_waves == 1)
+                    else if(B == 32 && minv_waves_ == 1)
                     {
                         // MFMA tiles: element (3 I + c / 3, 3 (I + dd) + c % 3) of the upper triangle
                         const int r = 3 * I + c / 3, col = 3 * (I + dd) + c % 3;

@@ -161,6 +161,7 @@ class Solver
     int  precision_  = kPrecFp32;
     int  entries_    = 4;
     int  mas_waves_  = 0;
+    int  minv_waves_ = 2;  // the local kernel whose layout the stored inverses are in
     int  effective_mas_waves() const;
     int  settable_variant(int waves) const;
     int  spmv_loads_ = 0;

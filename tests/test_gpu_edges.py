@@ -142,6 +142,33 @@ def test_lane_tiles_agree_with_the_block_diagonal_layout(bank, precision, n, con
         assert st["failure"] == 0 and st["rel_res_true"] <= 1e-4 * (1 + 1e-6)
 
 
+@pytest.mark.parametrize("bank,precision", [(32, "fp32"), (32, "fp16"), (16, "fp32"), (16, "bf16")])
+def test_inverse_is_read_in_the_layout_it_was_built_in(bank, precision):
+    """New values ask for a build, and another local kernel set before it does
+    not change how the inverses held are read (each kernel stores them in a
+    layout of its own); set with a build in place, it builds them again from
+    the same values."""
+    from agipc_learning_amd import session
+    from agipc_learning_amd import workloads as W
+
+    w = W.fem_grid(9, n_contacts=150, seed=3, young_sigma=0.5)
+    s = session.solver_for(w, bank=bank)
+    s.build(precision)
+    inv = s.inverse()
+    s.set_mas_waves(8)
+    assert np.array_equal(s.inverse(), inv)
+    s.set_mas_waves(0)
+    s.set_values(0, dev(3.0 * w["vals"]))
+    for waves in (4, 0, 8, 1):
+        s.set_mas_waves(waves)
+        assert np.array_equal(s.inverse(), inv), waves
+    r = dev(np.ones(3 * w["block_rows"]))
+    with pytest.raises(RuntimeError, match="build"):
+        s.apply_preconditioner(r, torch.zeros_like(r))
+    s.build(precision)
+    assert not np.array_equal(s.inverse(), inv)
+
+
 def mas_object(w, m=None, levels=0):
     """A preconditioner object of the mesh of w (or m given that mesh)."""
     from agipc_learning_amd import workloads as W
