@@ -447,6 +447,14 @@ int masx_set_mas_waves(masx_solver* s, int waves)
     });
 }
 
+int masx_mas_waves_used(masx_solver* s, int* waves)
+{
+    return guard([&] {
+        require(s != nullptr && waves != nullptr, "null argument");
+        *waves = s->impl.mas_waves_used();
+    });
+}
+
 int masx_autotune_mas(masx_solver* s, int reps, int* waves, double* ms)
 {
     return guard([&] {

@@ -125,7 +125,8 @@ class Solver
     // 4).  After a build, a change between the MFMA and the block-diagonal
     // layout leaves the solver unbuilt; one to or from lane tiles builds again.
     void set_mas_waves(int waves);
-    int  mas_waves() const { return settable_variant(mas_waves_); }
+    // the local kernel that runs: 0 lane tiles, else a variant's code
+    int  mas_waves_used() const { return mas_waves_ == 0 ? 0 : settable_variant(mas_waves_); }
     // times the settable MAS local variants of the built precision, returns the
     // fastest and sets it if it beats the automatic kernel
     Tiling autotune_mas(int reps);

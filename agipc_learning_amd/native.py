@@ -97,6 +97,7 @@ def load():
         "masx_morton_partition_device_noalloc": ([C.c_int, vp, C.c_int, vp, C.c_longlong, vp, vp], C.c_int),
         "masx_stream_rate": ([C.c_longlong, C.c_int, C.c_int, C.POINTER(C.c_double)], C.c_int),
         "masx_set_mas_waves": ([vp, C.c_int], C.c_int),
+        "masx_mas_waves_used": ([vp, C.POINTER(C.c_int)], C.c_int),
         "masx_set_spmv_loads": ([vp, C.c_int], C.c_int),
         "masx_set_factor_waves": ([vp, C.c_int], C.c_int),
         "masx_spmv_loads_used": ([vp, ip], C.c_int),
@@ -459,6 +460,12 @@ class Solver:
     def set_mas_waves(self, waves):
         check(self.L.masx_set_mas_waves(self.h, waves))
 
+    def mas_waves_used(self):
+        """The MAS local kernel that runs: 0 lane tiles, else a variant's code."""
+        w = C.c_int()
+        check(self.L.masx_mas_waves_used(self.h, C.byref(w)))
+        return w.value
+
     def set_factor_waves(self, waves):
         """MAS factor: 1 or 2 waves per bank, 0 automatic (next build)."""
         check(self.L.masx_set_factor_waves(self.h, waves))
@@ -496,11 +503,13 @@ class Solver:
         return out[:n.value]
 
     def autotune_mas(self, reps=50):
-        """Times every supported wave count of the MAS local kernel (built
-        precision) and keeps the fastest."""
+        """Times the MAS local variants that can be set (built precision).
+        `waves` and `ms` are the fastest of them; `used` is what runs
+        afterwards: that variant where it is more than 2 % faster than the
+        automatic kernel, else 0, the automatic one."""
         w, ms = C.c_int(), C.c_double()
         check(self.L.masx_autotune_mas(self.h, reps, C.byref(w), C.byref(ms)))
-        return dict(waves=w.value, ms=ms.value)
+        return dict(waves=w.value, ms=ms.value, used=self.mas_waves_used())
 
     def time_kernel(self, which, reps=20):
         ms = C.c_double()

@@ -209,6 +209,9 @@ int masx_spmv_loads_used(masx_solver* s, int* nontemporal);
  * 32-slot banks on, else as 4): that needs a new masx_build before the next
  * solve (masx_solve reports the missing build). */
 int masx_set_mas_waves(masx_solver* s, int waves);
+/* *waves: the MAS local kernel that runs with the current setting, 0 (lane
+ * tiles) or the code of a variant. */
+int masx_mas_waves_used(masx_solver* s, int* waves);
 /* MAS factor (the dense assembly and FP64 inverse of every bank at
  * masx_build): waves = 1, one wave per bank (more banks per SIMD; the faster
  * on many banks), 2, two waves per bank (a bank's inverse sooner; the faster
@@ -220,8 +223,9 @@ int masx_set_factor_waves(masx_solver* s, int waves);
 /* Times the MAS local variants of the built precision (`reps` launches
  * each; for half-precision 32-slot banks 1, 4 and 8, else 4, 8, 5 and 9),
  * reports the fastest of them and its time per launch (ms), and sets it if it
- * beats the automatic kernel (0), which stays otherwise; the preconditioner is
- * built again for a layout change.  Leaves the iteration state frozen like
+ * is more than 2 % faster than the automatic kernel (0), which is set otherwise
+ * (masx_mas_waves_used tells which); the preconditioner is built again for a
+ * layout change.  Leaves the iteration state frozen like
  * masx_autotune. */
 int masx_autotune_mas(masx_solver* s, int reps, int* waves, double* ms);
 /* Average execution time of one kernel (0 MAS local, 1 preconditioner finish,

@@ -169,6 +169,37 @@ def test_inverse_is_read_in_the_layout_it_was_built_in(bank, precision):
     assert not np.array_equal(s.inverse(), inv)
 
 
+@pytest.mark.parametrize("bank,precision", [(32, "fp32"), (32, "fp16"), (16, "fp32"), (16, "bf16")])
+def test_autotune_says_which_local_kernel_runs(bank, precision):
+    """After the autotuner the solver is built and applies, bit for bit, as one
+    set to the variant reported as used: the reported fastest or the automatic
+    kernel, whatever was set before."""
+    from agipc_learning_amd import session
+    from agipc_learning_amd import workloads as W
+
+    w = W.fem_grid(9, n_contacts=150, seed=3, young_sigma=0.5)
+    r = dev(np.random.default_rng(2).standard_normal(3 * w["block_rows"]))
+
+    def applied(s):
+        z = torch.zeros_like(r)
+        s.apply_preconditioner(r, z)
+        return host(z)
+
+    for before in (0, 4, 8, 1):
+        s = session.solver_for(w, bank=bank)
+        s.set_mas_waves(before)
+        s.build(precision)
+        if before == 0:
+            assert s.mas_waves_used() == 0
+        best = s.autotune_mas(3)
+        assert best["used"] == s.mas_waves_used() and best["used"] in (0, best["waves"])
+        other = session.solver_for(w, bank=bank)
+        other.set_mas_waves(best["used"])
+        other.build(precision)
+        assert other.mas_waves_used() == best["used"]
+        assert np.array_equal(applied(s), applied(other))
+
+
 def mas_object(w, m=None, levels=0):
     """A preconditioner object of the mesh of w (or m given that mesh)."""
     from agipc_learning_amd import workloads as W

@@ -475,7 +475,7 @@ def test_mas_waves_agree_and_autotune(oracle, bank):
     same preconditioner (the FP32 sums of the waves' partials in another
     order: within 1e-6 of each other, 1e-4 of the oracle's apply; the staged
     form of a wave count bit for bit like the unstaged one) and gives the
-    same solve; the autotuner keeps one of them."""
+    same solve; the autotuner reports one of them."""
     w = W.fem_grid(12, n_contacts=300, seed=21, young_sigma=0.5)
     s = session.solver_for(w, bank=bank)
     s.build("fp32")
@@ -507,7 +507,7 @@ def test_half_local_variants_agree_and_autotune(precision):
     the 4- and 8-wave VALU kernels (block-diagonal layout) apply the same
     stored inverse (FP32 accumulation in other orders: within 1e-5 of each
     other) and give the same solve; switching between the layouts asks for a
-    new build; the autotuner keeps one of the three."""
+    new build; the autotuner reports one of the three."""
     w = W.fem_grid(12, n_contacts=300, seed=22, young_sigma=0.5)
     s = session.solver_for(w)
     r = dev(np.random.default_rng(5).standard_normal(3 * w["block_rows"]))
