@@ -331,7 +331,7 @@ __global__ void __launch_bounds__(256) k_fem_element(int n_tets, const double* _
 // this; the scratch read with nontemporal loads was slower (584).
 constexpr int kGatherTargets = 32, kGatherChunk = 28 * 9;
 __global__ void __launch_bounds__(256) k_fem_gather(long long nb, const long long* __restrict__ ptr,
-                                                    const int* __restrict__ contrib, const double* __restrict__ elem,
+                                                    const uint32_t* __restrict__ contrib, const double* __restrict__ elem,
                                                     const double* __restrict__ base, double* __restrict__ vals)
 {
     constexpr int K = 9, OWN = (9 * kGatherTargets + 255) / 256;  // contributions in flight and sums per thread
@@ -366,8 +366,8 @@ __global__ void __launch_bounds__(256) k_fem_gather(long long nb, const long lon
 #pragma unroll 1
         for(int pass = g; pass < n && tid < 252; pass += 28 * K)
         {
-            int    code[K];
-            double v[K];
+            uint32_t code[K];
+            double   v[K];
 #pragma unroll
             for(int k = 0; k < K; ++k) code[k] = contrib[e0 + c0 + min(pass + 28 * k, n - 1)];
 #pragma unroll
@@ -509,7 +509,7 @@ FemHessian::~FemHessian()
 void FemHessian::setup(int n_tets, const int* tets, long long nb, const int* rows, const int* cols)
 {
     if(n_tets <= 0 || !tets) throw std::invalid_argument("no tets");
-    if(n_tets > (1 << 30) / kBlocksPerTet - 64) throw std::invalid_argument("too many tets");
+    if(n_tets > (1 << 30) / kBlocksPerTet) throw std::invalid_argument("too many tets");
     if(nb <= 0 || !rows || !cols) throw std::invalid_argument("empty block structure");
     int n_rows = 0;
     for(long long k = 0; k < nb; ++k)
@@ -547,7 +547,7 @@ void FemHessian::setup(int n_tets, const int* tets, long long nb, const int* row
     };
     // contributions (tet, a, b) with tets[a] <= tets[b], in tet order
     std::vector<long long> target;
-    std::vector<int>       code;
+    std::vector<uint32_t>  code;  // 32 bits: the slots of the last group of 64 tets may pass 2^30
     target.reserve((size_t)n_tets * kBlocksPerTet);
     code.reserve((size_t)n_tets * kBlocksPerTet);
     for(int t = 0; t < n_tets; ++t)
@@ -565,13 +565,13 @@ void FemHessian::setup(int n_tets, const int* tets, long long nb, const int* row
                 const long long j = find(p, q);
                 if(j < 0) throw std::invalid_argument("a tet edge or vertex has no block in the structure");
                 target.push_back(j);
-                code.push_back((elem_slot(t, tet_block(std::min(a, b), std::max(a, b))) << 1) | (a > b ? 1 : 0));
+                code.push_back(((uint32_t)elem_slot(t, tet_block(std::min(a, b), std::max(a, b))) << 1) | (a > b ? 1u : 0u));
             }
     }
     std::vector<long long> ptr(nb + 1, 0);
     for(long long j : target) ++ptr[j + 1];
     for(long long j = 0; j < nb; ++j) ptr[j + 1] += ptr[j];
-    std::vector<int>       sorted(code.size());
+    std::vector<uint32_t>  sorted(code.size());
     std::vector<long long> cur(ptr.begin(), ptr.end() - 1);
     for(size_t e = 0; e < code.size(); ++e) sorted[cur[target[e]]++] = code[e];
 
@@ -582,11 +582,11 @@ void FemHessian::setup(int n_tets, const int* tets, long long nb, const int* row
     d_contrib_ = nullptr;
     fem_check(hipMalloc((void**)&d_tets_, sizeof(int) * 4 * (size_t)n_tets));
     fem_check(hipMalloc((void**)&d_ptr_, sizeof(long long) * (nb + 1)));
-    fem_check(hipMalloc((void**)&d_contrib_, sizeof(int) * std::max<size_t>(1, sorted.size())));
+    fem_check(hipMalloc((void**)&d_contrib_, sizeof(uint32_t) * std::max<size_t>(1, sorted.size())));
     fem_check(hipMemcpy(d_tets_, tets, sizeof(int) * 4 * (size_t)n_tets, hipMemcpyHostToDevice));
     fem_check(hipMemcpy(d_ptr_, ptr.data(), sizeof(long long) * (nb + 1), hipMemcpyHostToDevice));
     if(!sorted.empty())
-        fem_check(hipMemcpy(d_contrib_, sorted.data(), sizeof(int) * sorted.size(), hipMemcpyHostToDevice));
+        fem_check(hipMemcpy(d_contrib_, sorted.data(), sizeof(uint32_t) * sorted.size(), hipMemcpyHostToDevice));
     n_tets_ = n_tets;
     nb_     = nb;
     n_rows_ = n_rows;

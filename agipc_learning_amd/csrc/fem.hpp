@@ -45,7 +45,7 @@ class FemHessian
     long long nb_ = 0;
     int*      d_tets_ = nullptr;     // 4 per tet
     long long* d_ptr_ = nullptr;     // nb + 1
-    int*      d_contrib_ = nullptr;  // scratch block << 1 | transposed
+    uint32_t* d_contrib_ = nullptr;  // scratch block << 1 | transposed
     double*   d_elem_ = nullptr;     // 10 blocks x 9 per tet (whole groups of 64 tets)
     size_t    elem_cap_ = 0;
 };

@@ -184,3 +184,20 @@ def test_spmv_layout_with_body_couplings(entries):
     body_full = int(in_bodies.sum() + (in_bodies & (rows != cols)).sum())
     assert err <= 1e-13
     assert n_ent == n + 2 * off - body_full - n_once
+
+
+@pytest.mark.parametrize("n_tets,says", [((1 << 30) // 10, "empty block structure"), ((1 << 30) // 10 - 63, "empty block structure"),
+                                         ((1 << 30) // 10 + 1, "too many tets")])
+def test_fem_accepts_tets_up_to_its_limit(n_tets, says):
+    """The count is checked before the structure, and both before any array is
+    read: (2^30) / 10 tets pass, one more does not.  The last group of 64 tets
+    then has scratch blocks past 2^30, which twice fit 32 bits unsigned."""
+    import ctypes as C
+
+    L = native.load()
+    one = np.zeros(4, np.int32).ctypes.data_as(C.POINTER(C.c_int))
+    h = C.c_void_p()
+    assert L.masx_fem_create(C.byref(h), n_tets, one, 0, one, one) != 0
+    assert says in L.masx_last_error().decode()
+    t = min(n_tets, (1 << 30) // 10) - 1
+    assert 2 * (((t >> 6) * 10 + 9) * 64 + (t & 63)) + 1 < 1 << 32
