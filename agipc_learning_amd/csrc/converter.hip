@@ -30,7 +30,13 @@ constexpr int kScanItems = 8;               // elements per thread in the block 
 constexpr int kScanTile  = kScanBlock * kScanItems;
 constexpr int kRowRegs   = 128;             // longest row sorted in registers (two keys per lane)
 constexpr int kRowCap    = 1024;            // longest row sorted in LDS; longer rows sort in global scratch
-constexpr int kLongGrid  = 1024;            // workgroups that walk the rows longer than kRowRegs
+// The rows longer than kRowRegs go to 64 lists (a workgroup's to the list of its
+// index), their counts a line apart, and at most 40 one-wave workgroups walk a
+// list: as many as the keys' LDS lets run at once.  20,000 rows of 200 triplets
+// in random order: 228 us of queueing at one list's counter and 691 of sorting
+// (1,024 workgroups, keys read by flat instructions), 8 and 160 now; a walk by
+// 16 workgroups a list takes 7-15 % longer over 140 to 1,000 triplets a row.
+constexpr int kLongLists = 64, kLongPerList = 40, kLongStride = 16;
 constexpr uint32_t kHead = 0x80000000u;     // bucket entry: first of its column run (an input index has 31 bits)
 constexpr uint32_t kNone = 0xffffffffu;     // rank of a triplet that is dropped
 
@@ -152,14 +158,16 @@ __global__ void __launch_bounds__(kScanBlock) k_scan_add(int* out, int m, const 
 // below.
 __global__ void __launch_bounds__(256) k_conv_row_sort(int nr, const int* __restrict__ row_start,
                                                        uint32_t* __restrict__ bucket, const int* __restrict__ cols,
-                                                       int* __restrict__ uniq, int* __restrict__ long_rows, int* n_long)
+                                                       int* __restrict__ uniq, int* __restrict__ long_rows,
+                                                       int list_cap, int* n_long)
 {
     const int r = blockIdx.x * 4 + (int)(threadIdx.x >> 6);
     if(r >= nr) return;
     const int rs = row_start[r], L = row_start[r + 1] - rs, lane = threadIdx.x & 63;
     if(L > kRowRegs)
     {
-        if(lane == 0) long_rows[atomicAdd(n_long, 1)] = r;
+        const int list = blockIdx.x % kLongLists;
+        if(lane == 0) long_rows[(size_t)list * list_cap + atomicAdd(&n_long[list * kLongStride], 1)] = r;
         return;
     }
     uint32_t t[2], c[2];
@@ -212,19 +220,19 @@ __global__ void __launch_bounds__(256) k_conv_row_sort(int nr, const int* __rest
 }
 
 // The rows longer than kRowRegs, one wavefront each, with the keys in LDS (or
-// global scratch past kRowCap).
-__global__ void __launch_bounds__(64) k_conv_row_sort_long(const int* __restrict__ long_rows, const int* n_long,
-                                                           const int* __restrict__ row_start, uint32_t* bucket,
-                                                           const int* __restrict__ cols, unsigned long long* gkeys,
-                                                           unsigned long long* gsorted, int* uniq)
+// global scratch past kRowCap): a lane ranks four of its keys at a time against
+// every key.  The two places are told apart outside the loops, so the LDS
+// reads are LDS instructions.
+__global__ void __launch_bounds__(64) k_conv_row_sort_long(const int* __restrict__ long_rows, int list_cap,
+                                                           const int* n_long, const int* __restrict__ row_start,
+                                                           uint32_t* bucket, const int* __restrict__ cols,
+                                                           unsigned long long* gkeys, unsigned long long* gsorted,
+                                                           int* uniq)
 {
     __shared__ unsigned long long s_keys[kRowCap], s_sorted[kRowCap];
-    const int lane = threadIdx.x, rows_left = *n_long;
-    for(int q = blockIdx.x; q < rows_left; q += gridDim.x)
-    {
-        const int r = long_rows[q], rs = row_start[r], L = row_start[r + 1] - rs;
-        unsigned long long* keys   = L <= kRowCap ? s_keys : gkeys + rs;
-        unsigned long long* sorted = L <= kRowCap ? s_sorted : gsorted + rs;
+    const int lane = threadIdx.x, list = blockIdx.x % kLongLists;
+    const int rows_left = n_long[list * kLongStride];
+    auto sort_row = [&](int r, int rs, int L, unsigned long long* keys, unsigned long long* sorted) {
         for(int i = lane; i < L; i += 64)
         {
             const uint32_t t = bucket[rs + i];
@@ -232,12 +240,26 @@ __global__ void __launch_bounds__(64) k_conv_row_sort_long(const int* __restrict
         }
         __syncthreads();
         // keys are distinct (the input index is part of the key): rank = position
-        for(int i = lane; i < L; i += 64)
+        for(int i = lane; i < L; i += 256)
         {
-            const unsigned long long k = keys[i];
-            int rank = 0;
-            for(int j = 0; j < L; ++j) rank += keys[j] < k;
-            sorted[rank] = k;
+            unsigned long long k[4];
+            int                rank[4];
+#pragma unroll
+            for(int h = 0; h < 4; ++h)
+            {
+                k[h]    = keys[min(i + 64 * h, L - 1)];
+                rank[h] = 0;
+            }
+#pragma unroll 4
+            for(int j = 0; j < L; ++j)
+            {
+                const unsigned long long o = keys[j];
+#pragma unroll
+                for(int h = 0; h < 4; ++h) rank[h] += o < k[h];
+            }
+#pragma unroll
+            for(int h = 0; h < 4; ++h)
+                if(i + 64 * h < L) sorted[rank[h]] = k[h];
         }
         __syncthreads();
         int count = 0;
@@ -251,6 +273,14 @@ __global__ void __launch_bounds__(64) k_conv_row_sort_long(const int* __restrict
         }
         if(lane == 0) uniq[r] = count;
         __syncthreads();  // the next row reuses the LDS
+    };
+    for(int q = blockIdx.x / kLongLists; q < rows_left; q += gridDim.x / kLongLists)
+    {
+        const int r = long_rows[(size_t)list * list_cap + q], rs = row_start[r], L = row_start[r + 1] - rs;
+        if(L <= kRowCap)
+            sort_row(r, rs, L, s_keys, s_sorted);
+        else
+            sort_row(r, rs, L, gkeys + rs, gsorted + rs);
     }
 }
 
@@ -369,12 +399,14 @@ int Converter::convert(int n, int n_block_rows, const int* rows, const int* cols
     if(n == 0) return 0;
     if(!rows || !cols || !vals || !out_rows || !out_cols || !out_vals) throw std::invalid_argument("null pointer");
     const int nr = n_block_rows;
-    // row counts, then the bad-index flag and the count of long rows (one clear)
-    grow(row_count_, row_count_cap_, (size_t)nr + 2);
+    // row counts, then the bad-index flag and the counts of the long rows' lists (one clear)
+    const size_t n_clear  = ((size_t)nr + 1 + kLongLists * kLongStride + 3) / 4 * 4;
+    const int    list_cap = (int)((grid_for(nr, 4) + kLongLists - 1) / kLongLists) * 4;
+    grow(row_count_, row_count_cap_, n_clear);
     grow(row_start_, row_start_cap_, (size_t)nr + 1);
     grow(uniq_, uniq_cap_, (size_t)nr);
     grow(out_start_, out_start_cap_, (size_t)nr + 1);
-    grow(long_rows_, long_rows_cap_, (size_t)nr);
+    grow(long_rows_, long_rows_cap_, (size_t)list_cap * kLongLists);
     grow(rank_, rank_cap_, (size_t)n);
     grow(bucket_, bucket_cap_, (size_t)n);
     grow(keys_, keys_cap_, (size_t)n);
@@ -382,16 +414,16 @@ int Converter::convert(int n, int n_block_rows, const int* rows, const int* cols
     if(!h_pinned_) CONV_HIP(hipHostMalloc((void**)&h_pinned_, 2 * sizeof(int), hipHostMallocDefault));
     int *flag = row_count_ + nr, *n_long = flag + 1;
 
-    CONV_HIP(hipMemsetAsync(row_count_, 0, sizeof(int) * ((size_t)nr + 2), st));
+    CONV_HIP(hipMemsetAsync(row_count_, 0, sizeof(int) * n_clear, st));
     hipLaunchKernelGGL(k_conv_count, dim3(grid_for(n, 256)), dim3(256), 0, st, n, nr, rows, cols, drop_lower,
                        row_count_, rank_, flag);
     CONV_HIP(hipGetLastError());
     scan(row_count_, row_start_, nr, st);
     hipLaunchKernelGGL(k_conv_scatter, dim3(grid_for(n, 256)), dim3(256), 0, st, n, rows, rank_, row_start_, bucket_);
     hipLaunchKernelGGL(k_conv_row_sort, dim3(grid_for(nr, 4)), dim3(256), 0, st, nr, row_start_, bucket_, cols, uniq_,
-                       long_rows_, n_long);
-    hipLaunchKernelGGL(k_conv_row_sort_long, dim3((unsigned)std::min(nr, kLongGrid)), dim3(64), 0, st, long_rows_,
-                       n_long, row_start_, bucket_, cols, keys_, sorted_, uniq_);
+                       long_rows_, list_cap, n_long);
+    const int per_list = std::min({list_cap, kLongPerList, n / kRowRegs + 1});  // no list holds more rows
+    hipLaunchKernelGGL(k_conv_row_sort_long, dim3((unsigned)(kLongLists * per_list)), dim3(64), 0, st, long_rows_, list_cap, n_long, row_start_, bucket_, cols, keys_, sorted_, uniq_);
     CONV_HIP(hipGetLastError());
     scan(uniq_, out_start_, nr, st);
     hipLaunchKernelGGL(k_conv_write, dim3(grid_for(nr, 4)), dim3(256), 0, st, nr, row_start_, bucket_, out_start_, cols,

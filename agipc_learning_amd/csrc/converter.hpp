@@ -25,7 +25,7 @@ class Converter
   private:
     void scan(const int* in, int* out, int m, hipStream_t st);
 
-    int*                row_count_ = nullptr;  // per row; then the bad-index flag and the long rows' count
+    int*                row_count_ = nullptr;  // per row; then the bad-index flag and the long rows' counts
     int*                row_start_ = nullptr;
     uint32_t*           rank_      = nullptr;  // per triplet: its place in its row's bucket
     uint32_t*           bucket_    = nullptr;

@@ -101,6 +101,23 @@ def test_converter_row_lengths(oracle, lengths, spread):
             assert np.array_equal(host(a), b)
 
 
+def test_converter_many_long_rows(oracle):
+    """More rows past the register sort than the lists' workgroups take at
+    once (47 rows a list, 40 workgroups), so a workgroup sorts several, with
+    rows past the LDS sort among them; bit for bit as the oracle."""
+    rng = np.random.default_rng(5)
+    lengths = 129 + np.arange(3000) % 7
+    lengths[[0, 1, 1500, 2990, 2999]] = 1025
+    r = rng.permutation(np.repeat(np.arange(3000), lengths)).astype(np.int32)
+    c = rng.integers(0, 60, len(r)).astype(np.int32)
+    v = rng.standard_normal((len(r), 9))
+    conv = native.Converter()
+    for _ in range(2):  # the counts are cleared between calls
+        got = conv.convert(dev(r), dev(c), dev(v), 3000)
+        for a, b in zip(got, oracle.convert_triplets(r, c, v, False)):
+            assert np.array_equal(host(a), b)
+
+
 @pytest.mark.parametrize("bank", [32, 16])
 @pytest.mark.parametrize("precision", ["fp32", "fp16", "bf16"])
 @pytest.mark.parametrize("n,contacts", [(2, 0), (3, 4), (9, 150)])
