@@ -101,6 +101,22 @@ def test_converter_row_lengths(oracle, lengths, spread):
             assert np.array_equal(host(a), b)
 
 
+@pytest.mark.parametrize("n_rows", [2047, 2048, 2049, 4097, 2048 * 256 + 1, 2048 * 300])
+def test_converter_scan_tiles(oracle, n_rows):
+    """Row counts around the prefix scan's tiles of 2,048 rows and past the 256
+    tiles that one pass over their totals takes; most rows are empty, the last one
+    is not.  Bit for bit as the oracle."""
+    rng = np.random.default_rng(n_rows)
+    n = 3 * min(n_rows, 20000)
+    r = rng.integers(0, n_rows, n).astype(np.int32)
+    r[:4] = n_rows - 1
+    c = np.minimum(r + rng.integers(0, 3, n), n_rows - 1).astype(np.int32)
+    v = rng.standard_normal((n, 9))
+    got = native.Converter().convert(dev(r), dev(c), dev(v), n_rows)
+    for a, b in zip(got, oracle.convert_triplets(r, c, v, False)):
+        assert np.array_equal(host(a), b)
+
+
 def test_converter_many_long_rows(oracle):
     """More rows past the register sort than the lists' workgroups take at
     once (47 rows a list, 40 workgroups), so a workgroup sorts several, with
@@ -116,6 +132,75 @@ def test_converter_many_long_rows(oracle):
         got = conv.convert(dev(r), dev(c), dev(v), 3000)
         for a, b in zip(got, oracle.convert_triplets(r, c, v, False)):
             assert np.array_equal(host(a), b)
+
+
+def clustered_system(n_banks, per_vertex, seed):
+    """Two slots to a level-1 node except the last 32 (all of one node, every
+    pair coupled); the level-1 nodes of fine banks 2j and 2j + 1 pair up, those of
+    banks 0 and 1 form one level-2 node, every pair coupled.  Besides, per_vertex
+    random blocks a slot, most of them near the diagonal.  Vertices in random order."""
+    n, rng = 32 * n_banks, np.random.default_rng(seed)
+    edges = [(v, v + 1) for v in range(0, n, 2)] + [(v, v + 1) for v in range(n - 32, n - 1)]
+    for j in range(0, n_banks, 2):
+        edges += [(32 * j + 2 * k, 32 * j + 32 + 2 * k) for k in range(16)]
+    edges += [(2 * k, 32 + 2 * ((k + 1) % 16)) for k in range(16)]
+    part_to_real = rng.permutation(n)
+    e = part_to_real[np.unique(np.array(edges), axis=0)]
+    e = np.concatenate([e, e[:, ::-1]])
+    e = e[np.lexsort((e[:, 1], e[:, 0]))]
+    num = np.bincount(e[:, 0], minlength=n)
+    start = np.concatenate([[0], np.cumsum(num)[:-1]])
+    r = np.repeat(np.arange(n), per_vertex)
+    c = np.where(rng.random(len(r)) < 0.75, r + rng.integers(-300, 301, len(r)), rng.integers(0, n, len(r)))
+    c = np.clip(c, 0, n - 1)
+    dense = [np.stack(np.triu_indices(m), 1) + o for m, o in ((64, 0), (32, n - 32))]
+    p = part_to_real[np.concatenate([np.stack([np.arange(n)] * 2, 1), np.stack([r, c], 1)] + dense)]
+    p = np.unique(np.sort(p, axis=1), axis=0)
+    p = p[rng.permutation(len(p))]
+    rows, cols = p[:, 0].astype(np.int32), p[:, 1].astype(np.int32)
+    vals = 0.1 * rng.standard_normal((len(p), 9))
+    d = rows == cols
+    m = vals[d].reshape(-1, 3, 3)
+    # diagonally dominant: every row's blocks are smaller in sum than its diagonal
+    load = np.bincount(rows, minlength=n) + np.bincount(cols, minlength=n)
+    vals[d] = (0.5 * (m + m.transpose(0, 2, 1)) + np.eye(3) * load[rows[d], None, None]).reshape(-1, 9)
+    return n, rows, cols, vals, (start, num, e[:, 1]), part_to_real, np.argsort(part_to_real)
+
+
+def test_galerkin_sums_of_large_levels(oracle):
+    """Coarse levels of at least 65,536 entries (the sums that pass through LDS
+    32 entries at a time) from fine and from coarse sources, as they are,
+    transposed and doubled, with an entry of several 252-source chunks at both and
+    counts that 32 does not divide: every bank's inverse equals the oracle's, which
+    forms the coarse blocks from the fine ones.  Bound as in the other inverse
+    tests, 2e-5 of a bank's largest value."""
+    n, rows, cols, vals, nbr, p2r, r2p = clustered_system(600, 5, 13)
+    s = native.Solver()
+    s.add_system(block_rows=n, rows=rows, cols=cols)
+    s.set_topology(0, *nbr, p2r, r2p)
+    s.setup()
+    s.set_values(0, dev(vals))
+    s.build("fp32")
+    mas = oracle.Mas(n, n, *nbr, p2r, r2p)
+    mas.reorder()
+    table = mas.hierarchy()["coarse_table"]
+    I, J = table[rows, 0], table[cols, 0]
+    for level in (1, 2):  # entries of the level and their sources
+        lo, hi = np.minimum(I, J), np.maximum(I, J)
+        pair, count = np.unique(np.stack([lo, hi], 1), axis=0, return_counts=True)
+        assert len(pair) >= 65536 and len(pair) % 32 and count.max() > 252 and count.mean() <= 32
+        if level == 1:
+            assert 0.2 < np.mean(I > J) < 0.8
+            up = dict(zip(table[:, 0], table[:, 1]))
+            I, J = (np.array([up[a] for a in pair[:, k]]) for k in (0, 1))
+            assert (I > J).any() and ((I == J) & (pair[:, 0] != pair[:, 1])).any()
+    mas.assemble(vals, rows, cols)
+    mas.invert(1)
+    got = s.inverse()
+    want = mas.inverse().reshape(got.shape[0], -1, 3, 3).transpose(0, 1, 3, 2).reshape(got.shape)
+    assert s.factor_status() == 0
+    scale = np.abs(want).max(axis=(1, 2), keepdims=True)
+    assert (np.abs(got - want) <= 2e-5 * scale).all()
 
 
 @pytest.mark.parametrize("bank", [32, 16])
