@@ -1543,11 +1543,12 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4,
 // tiles over an 8 x 8 grid of lanes: lane (ty, tx) holds element
 // (ty + 8 a, tx + 8 b) of every stored tile a >= b, 78 values of a 32-slot
 // bank in registers, and multiplies each by r of its column and, off the
-// diagonal tiles, by r of its row.  That is 144 FMAs and 20 loads of 16 bytes
-// per lane for a whole bank, where the block-diagonal kernels (k_mas_local)
-// spend ~1,450 wave instructions per bank on 4-byte loads, shuffles of every
-// transposed product and index arithmetic: on a few thousand banks those were
-// bound by VALU issue, not by their bytes.  The layout holds 5 % more than the
+// diagonal tiles, by r of its row.  That is 144 FMAs and 19 loads of 16 bytes
+// and two of 4 per lane for a whole bank (nine and three in 16 bits), 253 VALU
+// instructions in all, where the block-diagonal kernels (k_mas_local) spend
+// 1,300-1,500 per bank on 4-byte loads, shuffles of every transposed product
+// and index arithmetic: on a few thousand banks those were bound by VALU
+// issue, not by their bytes.  The layout holds 5 % more than the
 // FP32 block diagonals (19,968 B: diagonal tiles are whole) and 7 % less than
 // the MFMA tiles (9,984 B), and measured on 91,066 banks: FP32 296 us (staged
 // block diagonals 291-316), FP16 156 and BF16 150 (MFMA 190), so every size

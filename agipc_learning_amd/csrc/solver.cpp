@@ -1010,8 +1010,10 @@ void Solver::solve(const double* d_b, double* d_x, const SolveParams& prm, std::
     // one chunk later) the next chunk waits for the status of the one before.
     // A chunk launched past convergence is ~30 launches that exit at once,
     // 50-60 us before the result can be read (8^3 grid, FP32, 40 iterations:
-    // 1225 -> 1168 us a solve with its build); a wait costs ~10 us when the solve goes
+    // 1235 -> 1168 us a solve with its build); a wait costs ~10 us when the solve goes
     // on.  Further on the prediction has failed and chunks go out ahead again.
+    // The first kDepth chunks always go out at once, so after a solve of fewer
+    // iterations than they hold one still runs past the end.
     const int needed = last_iters_ > 0 ? last_iters_ / chunk + 1 : max_chunks;
     auto      depth  = [&] { return launched >= needed && launched < needed + 2 ? 1 : kDepth; };
     while(launched < ahead) launch_one();
